@@ -256,6 +256,137 @@ __global__ __launch_bounds__(kQT) void k_weight_rows_vec(const uint16_t* __restr
   }
 }
 
+// 8 bf16 over a finite scale s -> the bytes of quant8_div, in three operations per quotient instead of
+// the ten of the IEEE division sequence: y = 1 / s rounded, q = x y, then one residual step. The
+// quotient can be one fp32 unit off the correctly rounded one, its e4m3 code never is: over all
+// 1,065,402,240 pairs of a bf16 value and a bf16 maximum at or above its magnitude (every x and s
+// the quantizers can meet) the codes are equal, signs of zero included. x is finite (its row's or tensor's maximum is), and the
+// convert takes a quotient one unit above 448 to 448, as the clamp would.
+// (non-temporal: a 200 MB layer would leave the caches full of its dirty lines, and the next
+// matrix's reads wait for their eviction: one layer per channel 96.8 -> 92.3 us, the per-tensor
+// maximum pass after them 25 -> 19 us at gate_up)
+KRQ_DEV void st16nt(uint8_t* p, uint4 v) {
+  __builtin_nontemporal_store(v4u{v.x, v.y, v.z, v.w}, reinterpret_cast<v4u*>(p));
+}
+KRQ_DEV float quot(float x, float s, float y) {
+  const float q = x * y;
+  return fmaf(-fmaf(q, s, -x), y, q);  // (the residual's signs keep a quotient of -0)
+}
+KRQ_DEV uint2 quant8_quot(uint4 v, float s, float y) {
+  const uint32_t a[4] = {v.x, v.y, v.z, v.w};
+  int p[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t a0 = a[2 * h], a1 = a[2 * h + 1];
+    int q = __builtin_amdgcn_cvt_pk_fp8_f32(quot(as_f32(a0 << 16), s, y), quot(as_f32(a0 & 0xffff0000u), s, y), 0, false);
+    p[h] = __builtin_amdgcn_cvt_pk_fp8_f32(quot(as_f32(a1 << 16), s, y), quot(as_f32(a1 & 0xffff0000u), s, y), q, true);
+  }
+  return make_uint2(static_cast<uint32_t>(p[0]), static_cast<uint32_t>(p[1]));
+}
+
+// Weight rows in whole lines (N % 16 == 0, K % 64 == 0, 16-byte aligned rows): a workgroup of NW waves
+// owns eight rows (half a tile row); wave w takes their 128-element pieces w, w + NW, ... (C at most),
+// every one in registers between the maximum and the cast. Lane 8 p + r holds elements 16 p ..
+// 16 p + 15 of row r's piece, so each store writes whole 128-byte lines: one of each row of w8, and in
+// the tiled copy the eight adjacent 16-byte entries of rows 0-7 or 8-15. (One row per workgroup,
+// above, wrote each line of the tiled copy in 16-byte entries from eight workgroups on different
+// XCDs, and spent more time in IEEE divisions than in memory.)
+//   MODE 0 (per channel): the row's maximum over its lanes and the waves, then scale[n] and the cast
+//   MODE 1 (per tensor, pass 1): the workgroup takes row groups b, b + grid, ...; part[b] = their maximum
+//   MODE 2 (per tensor, pass 2): every workgroup folds the np partial maxima to the scale (block 0
+//          stores it) and casts its rows
+// Bound by HBM. A Qwen3-4B layer (202 MB in, 202 MB out; a device copy moves as much in 82 us) per
+// channel: 131.2 -> 92.5 us, of it gate_up 58 -> 40, down 25 -> 27, QKV 22 -> 15, O 15 -> 12; per
+// tensor, kernel times: gate_up 82 -> 51, down 32 -> 32, QKV 31 -> 17, O 20 -> 15 with one launch
+// fewer. Twice the waves with half the pieces each took 95.0 us, half the waves 100.0, whole 16-row
+// tiles 100.1.
+template <int MODE, int NW, int C>
+__global__ __launch_bounds__(NW * 64) void k_weight_lines(const uint16_t* __restrict__ w, int64_t K, int64_t ldw,
+                                                          uint8_t* __restrict__ w8, uint8_t* __restrict__ w8t,
+                                                          float* __restrict__ scale, float* __restrict__ part,
+                                                          int64_t groups, int np) {
+  __shared__ uint32_t red[NW][8];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int r = lane & 7, p = lane >> 3;
+  const int ne = static_cast<int>(K >> 4);  // 16-element entries of a row
+  uint4 v[C][2];
+  auto load = [&](int64_t rb) {
+    const uint8_t* row = reinterpret_cast<const uint8_t*>(w + (rb * 8 + r) * ldw);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {  // (an entry past the row repeats its last one)
+      const int64_t e = min(8 * (wave + NW * c) + p, ne - 1);
+      v[c][0] = MODE == 0 ? ld16nt(row + 32 * e) : ld16(row + 32 * e);
+      v[c][1] = MODE == 0 ? ld16nt(row + 32 * e + 16) : ld16(row + 32 * e + 16);
+    }
+  };
+  auto lane_max = [&]() {
+    u16x2 m{0, 0};
+#pragma unroll
+    for (int c = 0; c < C; ++c) m = absmax8_bits(v[c][1], absmax8_bits(v[c][0], m));
+    return bits_max_to_u32(m);
+  };
+  if constexpr (MODE == 1) {
+    uint32_t mb = 0;
+    for (int64_t rb = blockIdx.x; rb < groups; rb += gridDim.x) {
+      load(rb);
+      mb = umax32(mb, lane_max());
+    }
+    mb = wave_max_u32_dpp(mb);
+    if (lane == 0) red[wave][0] = mb;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int i = 0; i < NW; ++i) mb = umax32(mb, red[i][0]);
+      part[blockIdx.x] = as_f32(mb);
+    }
+    return;
+  }
+  const int64_t rb = blockIdx.x;
+  load(rb);
+  float s;
+  if constexpr (MODE == 0) {
+    uint32_t mb = lane_max();
+#pragma unroll
+    for (int o = 8; o < kWave; o <<= 1) mb = umax32(mb, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mb), o, kWave)));
+    if (lane < 8) red[wave][lane] = mb;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NW; ++i) mb = umax32(mb, red[i][r]);
+    s = scale_from_amax(clamp_min_nan(as_f32(mb), 1e-12f));
+    if (threadIdx.x < 8) scale[rb * 8 + threadIdx.x] = s;
+  } else {
+    uint32_t mb = 0;
+    for (int i = threadIdx.x; i < np; i += NW * 64) mb = umax32(mb, mag_bits(part[i]));
+    mb = wave_max_u32_dpp(mb);
+    if (lane == 0) red[wave][0] = mb;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NW; ++i) mb = umax32(mb, red[i][0]);
+    s = scale_from_amax(clamp_min_nan(as_f32(mb), 1e-12f));
+    if (rb == 0 && threadIdx.x == 0) scale[0] = s;
+  }
+  // rows with an infinite or NaN maximum take the division itself (0, NaN or NaN codes, as torch's)
+  const bool fin = __all((as_u32(s) & 0x7f800000u) != 0x7f800000u);
+  const float y = 1.0f / s;
+  const int64_t n = rb * 8 + r;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int e = 8 * (wave + NW * c) + p;
+    if (e >= ne) break;
+    uint2 lo, hi;
+    if (fin) {
+      lo = quant8_quot(v[c][0], s, y);
+      hi = quant8_quot(v[c][1], s, y);
+    } else {
+      lo = quant8_div(v[c][0], s);
+      hi = quant8_div(v[c][1], s);
+    }
+    const uint4 q = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    if (w8) st16nt(w8 + n * K + 16 * (int64_t)e, q);
+    if (w8t) st16nt(w8t + (((n >> 4) * (K >> 6) + (e >> 2)) * 64 + 16 * (e & 3) + (n & 15)) * 16, q);
+  }
+}
+
 // per-row activation scale (act_scale), and with x8 the per-token cast (quant_rows where K % 16 != 0)
 __global__ __launch_bounds__(kQT) void k_act_rows_vec(const uint16_t* __restrict__ x, int64_t M, int64_t K,
                                                       float headroom, float* amax, float* inv,
@@ -435,6 +566,9 @@ __global__ __launch_bounds__(kQT) void k_cast_fold_vec(const uint16_t* __restric
     *reinterpret_cast<uint2*>(x8 + 8 * i) = quant8(ld16(reinterpret_cast<const uint8_t*>(x) + 16 * i), iv);
 }
 
+constexpr int64_t kLineMaxK = 8 * 16 * 128;  // a row of k_weight_lines' largest variant
+constexpr int kLinePartials = 1024;        // partial maxima of its per-tensor pass
+
 bool vec_ok(const void* p, int64_t K, int64_t ld) {
   return K % 8 == 0 && ld % 8 == 0 && K <= kVecMaxK && aligned16(p);
 }
@@ -446,11 +580,40 @@ int grid_for(int64_t work, int per_block, int cap) {
   return static_cast<int>(g);
 }
 
+// the workgroups of a persistent launch over `work` items with the same number of items each (the
+// last may have fewer): at most cap
+int balanced_grid(int64_t work, int64_t cap) {
+  const int64_t rounds = (work + cap - 1) / cap;
+  return static_cast<int>((work + rounds - 1) / rounds);
+}
+
 }  // namespace
 
 // =============================================================================================
 // C ABI
 // =============================================================================================
+// k_weight_lines' shapes: whole tiles, 16-byte aligned rows and copies, rows in registers.
+// Other shapes keep the one-row-per-workgroup kernels.
+static bool lines_ok(const void* w, int64_t N, int64_t K, int64_t ldw, const void* w8, const void* w8t) {
+  return N % 16 == 0 && K % 64 == 0 && K <= kLineMaxK && ldw % 8 == 0 && aligned16(w) && aligned16(w8) &&
+         aligned16(w8t);
+}
+
+template <int MODE>
+static void launch_weight_lines(const void* w, int64_t N, int64_t K, int64_t ldw, void* w8, void* w8t, float* scale,
+                                float* part, int np, int grid, hipStream_t s) {
+  const int np8 = static_cast<int>((K + 127) / 128);  // 128-element pieces of a row
+#define KRQ_LINES(NW, C)                                                                                      \
+  hipLaunchKernelGGL((k_weight_lines<MODE, NW, C>), dim3(grid), dim3(NW * 64), 0, s, (const uint16_t*)w, K, ldw, \
+                     (uint8_t*)w8, (uint8_t*)w8t, scale, part, N / 8, np)
+  if (np8 <= 8) KRQ_LINES(4, 2);
+  else if (np8 <= 20) KRQ_LINES(4, 5);
+  else if (np8 <= 32) KRQ_LINES(8, 4);
+  else if (np8 <= 80) KRQ_LINES(8, 10);
+  else KRQ_LINES(8, 16);
+#undef KRQ_LINES
+}
+
 extern "C" int krq_quant_fp8_rows(const void* w_bf16, int64_t N, int64_t K, int64_t ldw, void* w8,
                                   void* w8_tiled, float* scale, void* stream) {
   KRQ_REQUIRE(w_bf16 && scale && (w8 || w8_tiled), "quant_fp8_rows: null pointer");
@@ -460,6 +623,11 @@ extern "C" int krq_quant_fp8_rows(const void* w_bf16, int64_t N, int64_t K, int6
   KRQ_REQUIRE(!w8_tiled || (N % 16 == 0 && K % 64 == 0),
               "quant_fp8_rows: tiled layout needs N %% 16 == 0 and K %% 64 == 0 (N=%lld K=%lld)",
               (long long)N, (long long)K);
+  if (lines_ok(w_bf16, N, K, ldw, w8, w8_tiled)) {
+    launch_weight_lines<0>(w_bf16, N, K, ldw, w8, w8_tiled, scale, nullptr, 0, static_cast<int>(N / 8),
+                           (hipStream_t)stream);
+    return krq_check_launch("quant_fp8_rows");
+  }
   const bool vec = vec_ok(w_bf16, K, ldw) && (!w8 || aligned16(w8));
   hipLaunchKernelGGL(vec ? k_weight_rows_vec<0> : k_weight_rows<0>, dim3(static_cast<unsigned>(N)),
                      dim3(kQT), 0, (hipStream_t)stream, (const uint16_t*)w_bf16, K, ldw, (uint8_t*)w8,
@@ -478,6 +646,12 @@ extern "C" int krq_quant_fp8_tensor(const void* w_bf16, int64_t N, int64_t K, in
               "quant_fp8_tensor: tiled layout needs N %% 16 == 0 and K %% 64 == 0 (N=%lld K=%lld)",
               (long long)N, (long long)K);
   hipStream_t s = (hipStream_t)stream;
+  if (lines_ok(w_bf16, N, K, ldw, w8, w8_tiled)) {
+    const int np = balanced_grid(N / 8, kLinePartials);  // (at most N / 8 partials, within row_amax_ws)
+    launch_weight_lines<1>(w_bf16, N, K, ldw, nullptr, nullptr, nullptr, row_amax_ws, 0, np, s);
+    launch_weight_lines<2>(w_bf16, N, K, ldw, w8, w8_tiled, scale0, row_amax_ws, np, static_cast<int>(N / 8), s);
+    return krq_check_launch("quant_fp8_tensor");
+  }
   const bool vec = vec_ok(w_bf16, K, ldw) && (!w8 || aligned16(w8));
   hipLaunchKernelGGL(vec ? k_weight_rows_vec<1> : k_weight_rows<1>, dim3(static_cast<unsigned>(N)),
                      dim3(kQT), 0, s, (const uint16_t*)w_bf16, K, ldw, nullptr, nullptr, nullptr,

@@ -139,6 +139,30 @@ def test_quantize_per_channel(dev, N, K):
     assert torch.equal(ref.view(torch.uint8), q[0].view(torch.uint8))
 
 
+# k_weight_lines: eight-row groups, 128-element pieces. K below one piece, a half last piece, the last
+# K of each register variant and the first of the next, a strided matrix, and (N or K not in whole tiles,
+# rows past its longest) the one-row kernels. Every row holds bf16 bit patterns of all magnitudes up to
+# its maximum, which runs over the binades, so quotients fall on both sides of the e4m3 midpoints.
+@pytest.mark.parametrize("N,K,pad", [(16, 64, 0), (48, 192, 8), (16, 1024, 0), (32, 1088, 0), (16, 2560, 64),
+                                     (16, 2624, 0), (16, 4096, 0), (16, 4160, 0), (16, 10240, 0), (16, 10304, 0),
+                                     (16, 16384, 0), (16, 16448, 0), (24, 128, 0), (16, 72, 0), (16, 128, 4)])
+@pytest.mark.parametrize("per_tensor", [False, True])
+def test_quantize_lines(dev, N, K, pad, per_tensor):
+    rng = np.random.default_rng(N + K + pad)
+    amax = (np.linspace(0x2000, 0x7F00, N).astype(np.int64) + rng.integers(0, 128, N))[:, None]
+    bits = rng.integers(0, 1 << 15, (N, K + pad)) % (amax + 1)
+    bits[:, K // 2] = amax[:, 0]  # (every row's maximum is in it)
+    bits = (bits | (rng.integers(0, 2, bits.shape) << 15)).astype(np.uint16)
+    bits[:, :2] = [0, 0x8000]     # +0 and -0 keep their signs
+    w = torch.from_numpy(bits.view(np.int16).copy()).view(torch.bfloat16).to(dev)[:, :K]
+    want8, want_s = (O.quantize_weight if per_tensor else O.quantize)(bits[:, :K])
+    q = (fp8.quantize_weight if per_tensor else fp8.quantize)(w)
+    assert np.array_equal(q[1].cpu().numpy(), want_s)
+    assert np.array_equal(u8(q[0]), want8)
+    if N % 16 == 0 and K % 64 == 0:
+        assert np.array_equal(q.tiled.cpu().numpy(), O.tile(want8))
+
+
 @pytest.mark.parametrize("N,K", [(64, 256), QKV])
 def test_quantize_weight_per_tensor(dev, N, K):
     w = weight(N, K, 13)
