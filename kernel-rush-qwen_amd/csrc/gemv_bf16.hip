@@ -22,7 +22,7 @@ namespace {
 // that gives up makes the block's partials NaN) and then reads act with agent-scope (sc1) loads,
 // and counts its exit. sy >= 0 / nwo > 0: the block's K split and its wave count, given (the
 // chained kernel's one-dimensional grid and common block size); waves past nwo end at once.
-template <int MT, int MODE, int LAYOUT, int ALGO, int U, int PB, bool CHAIN = false>
+template <int MT, int MODE, int LAYOUT, int ALGO, int U, int PB, bool XO, bool CHAIN = false>
 KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __restrict__ w, int M, int64_t NO,
                             int64_t K, int kts, void* __restrict__ out, void* __restrict__ aux, int64_t bx,
                             int sy = -1, int nwo = 0, const FusedArgs* fa = nullptr) {
@@ -30,6 +30,7 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
   __shared__ float ones[32];
   static_assert(PB == 1 || (MODE != KRQ_OUT_SWIGLU && ALGO != 2), "paired row blocks: MFMA, no SwiGLU");
   static_assert(PB == 1 || PB == 2 || PB == 4, "one, two or four row blocks per block");
+  static_assert(XO ? MT == 1 : ALGO != 2 || LAYOUT == KRQ_W_TILED, "one activation load per step: at most eight rows");
   static_assert(!CHAIN || (PB == 1 && (MODE == KRQ_OUT_SWIGLU || MODE == kOutSwiGluHalf || MODE == KRQ_OUT_PARTIAL)),
                 "chained MLP: SwiGLU first stage, partials second stage");
   constexpr bool WAITS = CHAIN && MODE == KRQ_OUT_PARTIAL;  // (second stage)
@@ -44,6 +45,7 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
   const int64_t tbase = (int64_t)sidx * kts;
   const int64_t rowb = 2 * K;
   const int jcount = wave < nsteps ? (nsteps - wave + nw - 1) / nw : 0;
+  constexpr bool RM = LAYOUT == KRQ_W_ROWMAJOR;  // loads of whole lines (w_line_chunk)
   if (threadIdx.x < 32) ones[threadIdx.x] = 1.0f;
   // weight set p: the up half of the SwiGLU, else the p-th row block of this block
   auto rbp = [&](int p) -> int64_t { return MODE == KRQ_OUT_SWIGLU && p == 1 ? rb + (NO >> 4) : rb + p; };
@@ -69,7 +71,15 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
     const int j = jcount > 0 ? wave + min(cc, jcount - 1) * nw : 0;
     const int64_t t0 = tbase + 2 * j;
     const int64_t t1 = (2 * j + 1 < kts) ? t0 + 1 : t0;
-    if constexpr (MODE == kOutSwiGluHalf) {
+    if constexpr (RM) {
+      const int64_t o = t0 * 64 + 16 * w_line_chunk(lane, 2 * j + 1 >= kts);
+#pragma unroll
+      for (int p = 0; p < P; ++p) {  // (a half-pair block: its eight gate rows, then the up rows)
+        const int64_t row = (MODE == kOutSwiGluHalf ? 8 * rb : 16 * rbp(p)) + (r & 7);
+        wl[p][u] = ld16nt(w + row * rowb + o);
+        wh[p][u] = ld16nt(w + (row + (MODE == kOutSwiGluHalf ? NO : 8)) * rowb + o);
+      }
+    } else if constexpr (MODE == kOutSwiGluHalf) {
       wl[0][u] = ld16nt(w_addr_hp<LAYOUT>(w, rb, NO, t0, rowb, lane));
       wh[0][u] = ld16nt(w_addr_hp<LAYOUT>(w, rb, NO, t1, rowb, lane));
     } else {
@@ -80,21 +90,30 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
       }
     }
   };
+  // The activations in whole lines too (XL), row by row as row-major weights; XO: one load per step, the
+  // lane columns c and c + 8 taking the two halves of row c's line.
+  constexpr bool XL = RM || ALGO != 2;
   auto load_x = [&](int u, int cc) {
     const int j = jcount > 0 ? wave + min(cc, jcount - 1) * nw : 0;
     const int64_t t0 = tbase + 2 * j;
     const int64_t t1 = (2 * j + 1 < kts) ? t0 + 1 : t0;
+    const int64_t o = t0 * 64 + 16 * w_line_chunk(lane, 2 * j + 1 >= kts);
+    auto ld = [&](int m, int64_t a) -> uint4 {
+      if constexpr (WAITS)
+        return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             xrs, static_cast<int>(m * rowb) + static_cast<int>(a), 0, 16));
+      else
+        return ld16(x + m * rowb + a);
+    };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      const int m = ALGO == 2 ? 0 : min(mt * 16 + r, M - 1);
-      if constexpr (WAITS) {
-        const int o = static_cast<int>((int64_t)m * rowb + g * 16);
-        xl[u][mt] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xrs, o + static_cast<int>(t0 * 64), 0, 16));
-        xh[u][mt] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xrs, o + static_cast<int>(t1 * 64), 0, 16));
+      if constexpr (!XL) {  // (one row)
+        xl[u][mt] = ld(0, t0 * 64 + g * 16);
+        xh[u][mt] = ld(0, t1 * 64 + g * 16);
       } else {
-        const uint8_t* xr = x + (int64_t)m * rowb + g * 16;
-        xl[u][mt] = ld16(xr + t0 * 64);
-        xh[u][mt] = ld16(xr + t1 * 64);
+        const int m = ALGO == 2 ? 0 : mt * 16 + (r & 7);
+        xl[u][mt] = ld(min(m, M - 1), o);
+        if constexpr (!XO) xh[u][mt] = ld(min(m + 8, M - 1), o);
       }
     }
   };
@@ -105,17 +124,27 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
   auto consume_slot = [&](int u, int cc) {
     const int j = jcount > 0 ? wave + min(cc, jcount - 1) * nw : 0;
     const bool ok = cc < jcount, hi = ok && (2 * j + 1 < kts);
+    uint4 al[MT], ah[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      al[mt] = xl[u][mt];
+      ah[mt] = xh[u][mt];
+      if constexpr (XL) lines_to_tiles(xl[u][mt], XO ? xl[u][mt] : xh[u][mt], &al[mt], &ah[mt]);
+    }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      const uint4 bl = sel4(ok, wl[p][u]), bh = sel4(hi, wh[p][u]);
+      uint4 bl = wl[p][u], bh = wh[p][u];
+      if constexpr (RM) lines_to_tiles(wl[p][u], wh[p][u], &bl, &bh);
+      bl = sel4(ok, bl);
+      bh = sel4(hi, bh);
       if (ALGO == 2) {
-        sv[p][0] = dot8_bf16(bl, xl[u][0], sv[p][0]);
-        sv[p][1] = dot8_bf16(bh, xh[u][0], sv[p][1]);
+        sv[p][0] = dot8_bf16(bl, al[0], sv[p][0]);
+        sv[p][1] = dot8_bf16(bh, ah[0], sv[p][1]);
       } else {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          acc[p][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_v8bf(xl[u][mt]), as_v8bf(bl), acc[p][mt], 0, 0, 0);
-          acc[p][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_v8bf(xh[u][mt]), as_v8bf(bh), acc[p][mt], 0, 0, 0);
+          acc[p][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_v8bf(al[mt]), as_v8bf(bl), acc[p][mt], 0, 0, 0);
+          acc[p][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_v8bf(ah[mt]), as_v8bf(bh), acc[p][mt], 0, 0, 0);
         }
       }
     }
@@ -200,26 +229,26 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
   if constexpr (CHAIN) chain_tail<!WAITS>(*fa);
 }
 
-template <int MT, int MODE, int LAYOUT, int ALGO, int U, int PB>
+template <int MT, int MODE, int LAYOUT, int ALGO, int U, int PB, bool XO = false>
 __global__ __launch_bounds__(512) void k_gemv_bf16(const uint8_t* __restrict__ x,
                                                   const uint8_t* __restrict__ w, int M, int64_t NO,
                                                   int64_t K, int kts, void* __restrict__ out,
                                                   void* __restrict__ aux) {
-  gemv_bf16_body<MT, MODE, LAYOUT, ALGO, U, PB>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
+  gemv_bf16_body<MT, MODE, LAYOUT, ALGO, U, PB, XO>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
 }
 
 // The SwiGLU with its last column blocks split in half, as k_gemv_fp8_swiglu_mixed: workgroups
 // below nfull are two-matrix blocks, workgroup nfull + j is half-pair block 2 nfull + j (the same
 // steps per wave, so the same output bits).
-template <int LAYOUT, int ALGO, int U>
+template <int LAYOUT, int ALGO, int U, bool XO = false>
 __global__ __launch_bounds__(512) void k_gemv_bf16_swiglu_mixed(const uint8_t* __restrict__ x,
                                                                const uint8_t* __restrict__ w, int M, int64_t NO,
                                                                int64_t K, int kts, void* __restrict__ out,
                                                                void* __restrict__ aux, int nfull) {
   if (static_cast<int>(blockIdx.x) < nfull)
-    gemv_bf16_body<1, KRQ_OUT_SWIGLU, LAYOUT, ALGO, U, 1>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
+    gemv_bf16_body<1, KRQ_OUT_SWIGLU, LAYOUT, ALGO, U, 1, XO>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
   else
-    gemv_bf16_body<1, kOutSwiGluHalf, LAYOUT, ALGO, U, 1>(x, w, M, NO, K, kts, out, aux,
+    gemv_bf16_body<1, kOutSwiGluHalf, LAYOUT, ALGO, U, 1, XO>(x, w, M, NO, K, kts, out, aux,
                                                           (int64_t)blockIdx.x + nfull);
 }
 
@@ -230,7 +259,7 @@ __global__ __launch_bounds__(512) void k_gemv_bf16_swiglu_mixed(const uint8_t* _
 // of K split p / nrb2. Each stage keeps the standalone launch's plan, so act and the partials are
 // those of the two launches, bit for bit. The block holds max(NWG, NWD) waves; the waves a stage
 // does not use end at once (a barrier waits only for the waves that have not ended).
-template <int MT, int LAYOUT, int ALGO, int U>
+template <int MT, int LAYOUT, int ALGO, int U, bool XO>
 __global__ __launch_bounds__(512) void k_mlp_chain_bf16(const uint8_t* __restrict__ x, const uint8_t* __restrict__ wgu,
                                                        const uint8_t* __restrict__ wd, int M, int64_t I, int64_t H,
                                                        int kts_g, int kts_d, int nfull, int nrb2, int nwg, int nwd,
@@ -238,14 +267,14 @@ __global__ __launch_bounds__(512) void k_mlp_chain_bf16(const uint8_t* __restric
                                                        FusedArgs fa) {
   const int w = static_cast<int>(blockIdx.x);
   if (w < nfull) {
-    gemv_bf16_body<MT, KRQ_OUT_SWIGLU, LAYOUT, ALGO, U, 1, true>(x, wgu, M, I, H, kts_g, act, nullptr, w, 0, nwg, &fa);
+    gemv_bf16_body<MT, KRQ_OUT_SWIGLU, LAYOUT, ALGO, U, 1, XO, true>(x, wgu, M, I, H, kts_g, act, nullptr, w, 0, nwg, &fa);
   } else if (w < fa.n_first) {
     if constexpr (MT == 1)
-      gemv_bf16_body<1, kOutSwiGluHalf, LAYOUT, ALGO, U, 1, true>(x, wgu, M, I, H, kts_g, act, nullptr,
+      gemv_bf16_body<1, kOutSwiGluHalf, LAYOUT, ALGO, U, 1, XO, true>(x, wgu, M, I, H, kts_g, act, nullptr,
                                                                   (int64_t)w + nfull, 0, nwg, &fa);
   } else {
     const int p = w - fa.n_first;
-    gemv_bf16_body<MT, KRQ_OUT_PARTIAL, LAYOUT, ALGO, U, 1, true>(reinterpret_cast<const uint8_t*>(act), wd, M, H, I,
+    gemv_bf16_body<MT, KRQ_OUT_PARTIAL, LAYOUT, ALGO, U, 1, XO, true>(reinterpret_cast<const uint8_t*>(act), wd, M, H, I,
                                                                   kts_d, part, nullptr, p % nrb2, p / nrb2, nwd, &fa);
   }
 }
@@ -360,10 +389,11 @@ void launch(int M, int pb, dim3 grid, int nw, size_t smem, hipStream_t s, const 
   const dim3 block(nw * 64);
   constexpr int PB2 = MODE == KRQ_OUT_SWIGLU ? 1 : 2;
   constexpr int PB4 = MODE == kOutArgmax ? 4 : 1;  // (pb is 4 only for the argmax epilogue)
+  constexpr bool RM = LAYOUT == KRQ_W_ROWMAJOR;
   if (M == 1)
-    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 2, 4, 1>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
+    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 2, 4, 1, RM>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
   else if (M <= 4)
-    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 1, 4, 1>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
+    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 1, 4, 1, true>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
   else if (M <= 16 && pb == 4)
     hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 1, 2, PB4>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
   else if (M <= 16 && pb == 2)
@@ -398,10 +428,10 @@ bool launch_swiglu_mixed(int layout, int M, int64_t NO, int nw, size_t smem, hip
   const dim3 grid(static_cast<unsigned>(nfull + 2 * rem), 1), block(nw * 64);
 #define KRQ_BF16_MIXED(LAYOUT)                                                                                   \
   if (M == 1)                                                                                                    \
-    hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT, 2, 4>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
+    hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT, 2, 4, LAYOUT == KRQ_W_ROWMAJOR>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
                        nullptr, nfull);                                                                          \
   else if (M <= 4)                                                                                               \
-    hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT, 1, 4>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
+    hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT, 1, 4, true>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
                        nullptr, nfull);                                                                          \
   else                                                                                                           \
     hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT, 1, 2>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
@@ -541,14 +571,14 @@ extern "C" int krq_mlp_chain_bf16(const void* x, const void* w_gu, const void* w
   const uint8_t* gb = (const uint8_t*)w_gu;
   const uint8_t* db = (const uint8_t*)w_down;
   const int m = static_cast<int>(M);
-#define KRQ_CHAIN(MT_, LAYOUT, ALGO, U_)                                                                          \
-  hipLaunchKernelGGL((k_mlp_chain_bf16<MT_, LAYOUT, ALGO, U_>), grid, block, smem, s, xb, gb, db, m, I, H, kts_g, \
+#define KRQ_CHAIN(MT_, LAYOUT, ALGO, U_, XO_)                                                                        \
+  hipLaunchKernelGGL((k_mlp_chain_bf16<MT_, LAYOUT, ALGO, U_, XO_>), grid, block, smem, s, xb, gb, db, m, I, H, kts_g, \
                      kts_d, static_cast<int>(nfull), static_cast<int>(nrb2), nwg, nwd, (uint16_t*)act, (float*)out, fa)
 #define KRQ_CHAIN_M(LAYOUT)                          \
-  if (M == 1) KRQ_CHAIN(1, LAYOUT, 2, 4);            \
-  else if (M <= 4) KRQ_CHAIN(1, LAYOUT, 1, 4);       \
-  else if (M <= 16) KRQ_CHAIN(1, LAYOUT, 1, 2);      \
-  else KRQ_CHAIN(2, LAYOUT, 1, 2);
+  if (M == 1) KRQ_CHAIN(1, LAYOUT, 2, 4, LAYOUT == KRQ_W_ROWMAJOR);            \
+  else if (M <= 4) KRQ_CHAIN(1, LAYOUT, 1, 4, true);       \
+  else if (M <= 16) KRQ_CHAIN(1, LAYOUT, 1, 2, false);      \
+  else KRQ_CHAIN(2, LAYOUT, 1, 2, false);
   if (w_layout == KRQ_W_TILED) {
     KRQ_CHAIN_M(KRQ_W_TILED)
   } else {

@@ -116,6 +116,31 @@ KRQ_DEV const uint8_t* w_addr(const uint8_t* w, int64_t rb, int64_t t, int64_t r
   return w + (rb * 16 + (lane & 15)) * row_bytes + t * 64 + (lane >> 4) * 16;
 }
 
+// Row-major weights in whole lines. w_addr's lane order takes 64 bytes of sixteen rows per load, so each
+// 128-byte line of a row-major matrix goes through the caches twice, half a line at a time. Here a
+// step's first load takes the whole lines of rows 0-7 of the sixteen and its second those of rows
+// 8-15: lane column c reads row c % 8 and 16-byte chunk g + 4 (c / 8) of the step (w_line_chunk).
+// lines_to_tiles then gives every lane the bytes w_addr would have: lanes c and c ^ 8 exchange one
+// 16-byte register each (lanes 8-15 take the second load's low half of the line, lanes 0-7 the first
+// load's high half), one DPP move per dword. half: the step holds its low tile only (the high
+// chunks repeat the low ones; the consumer masks them).
+// Measured on row-major bf16 weights (four Qwen3-4B layers in one graph; on tiled copies of them 174
+// us at M = 1 and 215 at M = 16): M = 1 238.6 -> 187.0 us, M = 16 293.5 -> 237.4, M = 32 398 -> 337.
+// The activation rows of the matrix-core kernels are read the same way: M = 32 361 -> 337, and with
+// tiled weights 331 -> 295. Rings of four and five slots instead of two measured slower (M = 16
+// 256 and 258 against 246 us in one run).
+KRQ_DEV int w_line_chunk(int lane, bool half) { return (lane >> 4) + (half ? 0 : 4 * ((lane >> 3) & 1)); }
+
+template <int BANKS>
+KRQ_DEV uint32_t take_ror8(uint32_t own, uint32_t other) {  // lanes of BANKS: lane ^ 8's `other`
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(own), static_cast<int>(other), 0x128, 0xf,
+                                                           BANKS, false));
+}
+KRQ_DEV void lines_to_tiles(uint4 a, uint4 b, uint4* low, uint4* high) {
+  *low = make_uint4(take_ror8<0xc>(a.x, b.x), take_ror8<0xc>(a.y, b.y), take_ror8<0xc>(a.z, b.z), take_ror8<0xc>(a.w, b.w));
+  *high = make_uint4(take_ror8<0x3>(b.x, a.x), take_ror8<0x3>(b.y, a.y), take_ror8<0x3>(b.z, a.z), take_ror8<0x3>(b.w, a.w));
+}
+
 // The B-operand address of folded one-row block b (kOutResidualFold): lane column c = lane % 16
 // reads output row 4 b + c % 4 at tile t of quarter c / 4 of K (qt 64-byte tiles per quarter).
 template <int LAYOUT>

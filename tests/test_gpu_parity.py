@@ -800,6 +800,27 @@ def test_bf16_tiled_layout_matches_rowmajor(dev):
     assert getattr(wt, "krq_tiled", None) is None
 
 
+# Row-major weights and activations are loaded in whole lines and exchanged between lanes into the tiles'
+# operands: the packed copy's results bit for bit, at an odd tile count per split (a half last step),
+# one row, at most four (one activation load per step), either side of a half and a whole 16-row tile,
+# and on the mixed SwiGLU launch's half-pair blocks (N / 2 = 8,208 columns, over 512 row blocks).
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 9, 16, 17, 24, 25, 32])
+@pytest.mark.parametrize("N,K,split,swiglu", [(32, 96, 1, False), (32, 96, 3, False), (48, 2560, 2, False),
+                                              (32, 160, 1, True), (16416, 96, 1, True), (65568, 64, 1, False)])
+def test_bf16_line_loads_equal_tiles(dev, M, N, K, split, swiglu):
+    from kernels import gemv as G
+    x, w = act(M, K, 60 + M).to(dev), weight(N, K, 61).to(dev)
+    got = G.gemv_swiglu(x, w) if swiglu else G.gemv(x, w, split)
+    G.pack(w)
+    assert torch.equal(got, G.gemv_swiglu(x, w) if swiglu else G.gemv(x, w, split))
+    ref = (x.double() @ w.double().t()).cpu()
+    if swiglu:
+        g, u = ref[:, :N // 2].to(torch.bfloat16).double(), ref[:, N // 2:].to(torch.bfloat16).double()
+        ref = torch.nn.functional.silu(g).to(torch.bfloat16).double() * u
+    y = got.double().cpu()
+    assert rel_err(y.sum(0) if split > 1 else y, ref) <= TOL
+
+
 @pytest.mark.parametrize("M", [1, 16])
 def test_lmhead_bf16_tiled(dev, M):
     from kernels import gemv as G
