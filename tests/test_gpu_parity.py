@@ -101,6 +101,38 @@ def test_act_scale_and_cast(dev):
     assert z.amax.item() == np.float32(1e-6)
 
 
+# The casts take 16 values per piece, without the NaN-keeping clamp where a piece is finite: a piece
+# with a NaN or an infinity beside finite ones, products past 448 (headroom and inverses below the
+# maximum's), zero, negative, infinite and NaN inverses, per-row inverses, one piece, a partial last
+# round of pieces, and the eight-value (K % 16 == 8) and scalar kernels.
+@pytest.mark.parametrize("M,K", [(1, 16), (3, 2560), (17, 4112), (5, 200), (2, 100), (300, 9728)])
+def test_cast_pieces(dev, M, K):
+    x = act(M, K, 70 + M, 3.0)
+    clean = x.to(dev)
+    for headroom in (0.5, 1.0, 4.0):
+        a, y = fp8._act_scale_cast(clean, headroom)
+        b = fp8.ActScale(clean, headroom)
+        assert torch.equal(a.inv, b.inv) and torch.equal(a.scale, b.scale) and torch.equal(a.amax, b.amax)
+        assert np.array_equal(u8(y), O.cast(u16(x), b.inv.cpu().numpy()[0]))
+    x[0, 3], x[M - 1, K - 1], x[M // 2, K // 2], x[0, 0] = float("nan"), float("-inf"), -0.0, -float("nan")
+    xd = x.to(dev)
+    for inv in (1.0, 200.0, 0.0, -30.0, float("inf"), float("nan")):
+        iv = torch.tensor([inv], dtype=torch.float32)
+        ref = u8((x.float() * iv).clamp(-448, 448).to(torch.float8_e4m3fn))
+        assert np.array_equal(u8(fp8._cast_hip(xd, fp8.SharedScale(iv.to(dev), None))), ref), inv
+        if K % 64 == 0:
+            pad = np.zeros(((M + 15) // 16 * 16, K), np.uint8)
+            pad[:M] = ref
+            got = fp8.cast_tiled(xd, fp8.SharedScale(iv.to(dev), None))
+            assert np.array_equal(got.cpu().numpy(), O.tile(pad).reshape(-1)), inv
+    rows = torch.linspace(0.5, 300.0, M)
+    rows[M // 2] = float("inf")
+    y = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=dev)
+    rd = rows.to(dev)
+    L.call("krq_cast_fp8", L.ptr(xd), M, K, L.ptr(rd), 1, L.ptr(y), L.stream(xd))
+    assert np.array_equal(u8(y), u8((x.float() * rows[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn)))
+
+
 # 512-thread kernel (K % 16 == 0, up to its 16,384 maximum), 8-value chunk kernel (K % 16 == 8),
 # scalar kernel (K % 8 != 0, and rows longer than the vector kernels hold)
 @pytest.mark.parametrize("M,K", [(1, 2560), (16, 9728), (32, 4096), (3, 64), (2, 16384), (2, 200), (3, 100),
