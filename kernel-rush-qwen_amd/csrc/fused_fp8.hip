@@ -20,26 +20,26 @@ constexpr size_t kMaxSmem = 60 * 1024;
 // largest bf16 x slice (bytes) a block normalizes in its prologue (as in fused_gemv.hip)
 constexpr int64_t kNormStageMax = 24 * 1024;
 
-// RMSNorm + per-token e4m3 quantization of whole rows (one block of NT threads per row, K % 16 == 0,
-// K <= kRowMaxK): x8 = e4m3(h * inv), xs = amax(h) / 448 with the ActScale arithmetic of quant_rows
-// (amax floored at 1e-6), h = RMSNorm(x) * ln as every normalizing kernel computes it. Each wave
-// sums the row's sum-of-squares partials itself in the canonical order (lane l takes t = l, l + 64,
-// ..., SC per lane) instead of staging them in LDS, each thread holds 16-value pieces (two 16-byte
-// loads of x and of ln, one 16-byte store), and the amax is DPP wave maxima and one barrier.
-// Measured on MI355X (fused FP8 layer, M = 16, against 256 threads of 8-value chunks with the
-// partials staged in LDS and four barriers): gate_up + RMSNorm 15.01 -> 14.90 us, QKV + RMSNorm
-// 9.29 -> 9.09 us. TILED: x8 in the tiled activation layout (tiled_offset), one block per row of
-// the M rows padded to a multiple of 16, the pad rows zero. ROWSUM (one row): the row's own chunk
-// sums (sumsq8, chunk i = elements 8 i ..) staged in LDS, and each wave takes the canonical sum over
-// them instead of over ss_in.
+// RMSNorm + per-token e4m3 quantization of whole rows (one block of NT threads per row, C pieces per
+// thread, K % 16 == 0, K <= kRowMaxK): x8 = e4m3(h * inv), xs = amax(h) / 448 with the ActScale
+// arithmetic of quant_rows (amax floored at 1e-6), h = RMSNorm(x) * ln as every normalizing kernel
+// computes it. Each wave sums the row's sum-of-squares partials itself in the canonical order (lane l
+// takes t = l, l + 64, ..., SC per lane) instead of staging them in LDS, each thread holds 16-value
+// pieces (two 16-byte loads of x and of ln, one 16-byte store), and the amax is DPP wave maxima and
+// one barrier. It is a chain of latencies: with the row's sum by lane swaps instead of shuffles
+// (wave_sum), the convert without the NaN-keeping clamp and, up to 4,096 elements, one piece per
+// thread of 256 instead of two (most of them repeats) per thread of 512, the fused FP8 layer over
+// eight layers takes 324.4 instead of 343.3 us at M = 16. TILED: x8 in the tiled activation layout
+// (tiled_offset), one block per row of the M rows padded to a multiple of 16, the pad rows zero.
+// ROWSUM (one row): the row's own chunk sums (sumsq8, chunk i = elements 8 i ..) staged in LDS, and
+// each wave takes the canonical sum over them instead of over ss_in.
 constexpr int kNqThreads = 512;
-template <int NT, int SC, bool TILED, bool ROWSUM>
+template <int NT, int C, int SC, bool TILED, bool ROWSUM>
 __global__ __launch_bounds__(NT) void k_rmsnorm_quant_rows(const uint16_t* __restrict__ x,
                                                            const float* __restrict__ ss_in,
                                                            const uint16_t* __restrict__ ln, float eps,
                                                            int64_t M, int64_t K, uint8_t* __restrict__ x8,
                                                            float* __restrict__ xs) {
-  constexpr int C = kRowMaxK / 16 / NT;
   __shared__ uint32_t red[NT / 64];
   __shared__ float sq[ROWSUM ? kRowMaxK / 8 : 1];
   const int64_t m = blockIdx.x;
@@ -105,8 +105,8 @@ __global__ __launch_bounds__(NT) void k_rmsnorm_quant_rows(const uint16_t* __res
   for (int c = 0; c < C; ++c) {
     const int64_t e = 16 * (int64_t)(threadIdx.x + c * NT);
     if (e < K) {
-      const uint2 lo = quant8(v[c][0], iv), hi = quant8(v[c][1], iv);
-      *reinterpret_cast<uint4*>(x8 + (TILED ? tiled_offset(m, e, K) : m * K + e)) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      *reinterpret_cast<uint4*>(x8 + (TILED ? tiled_offset(m, e, K) : m * K + e)) =
+          quant16_own_amax(v[c][0], v[c][1], b, iv);
     }
   }
 }
@@ -115,16 +115,16 @@ template <bool TILED>
 void launch_rmsnorm_quant(int64_t rows, const void* x, const float* ss_in, const void* ln, float eps, int64_t M,
                           int64_t K, void* x8, float* x_scale, hipStream_t s) {
   // SC partials per lane: T = K / 16 <= 64 * SC; one row sums itself (ROWSUM)
-  const dim3 g(static_cast<unsigned>(rows)), b(kNqThreads);
-  if (M == 1)
-    hipLaunchKernelGGL((k_rmsnorm_quant_rows<kNqThreads, 1, TILED, true>), g, b, 0, s, (const uint16_t*)x, ss_in,
-                       (const uint16_t*)ln, eps, M, K, (uint8_t*)x8, x_scale);
-  else if (K <= 4096)
-    hipLaunchKernelGGL((k_rmsnorm_quant_rows<kNqThreads, 4, TILED, false>), g, b, 0, s, (const uint16_t*)x, ss_in,
-                       (const uint16_t*)ln, eps, M, K, (uint8_t*)x8, x_scale);
-  else
-    hipLaunchKernelGGL((k_rmsnorm_quant_rows<kNqThreads, kRowMaxK / 16 / 64, TILED, false>), g, b, 0, s,
-                       (const uint16_t*)x, ss_in, (const uint16_t*)ln, eps, M, K, (uint8_t*)x8, x_scale);
+  // (a row of up to 4,096 elements: one piece per thread of 256)
+  const dim3 g(static_cast<unsigned>(rows));
+#define KRQ_NQ(NT, C, SC, ROWSUM)                                                                                   \
+  hipLaunchKernelGGL((k_rmsnorm_quant_rows<NT, C, SC, TILED, ROWSUM>), g, dim3(NT), 0, s, (const uint16_t*)x, ss_in, \
+                     (const uint16_t*)ln, eps, M, K, (uint8_t*)x8, x_scale)
+  constexpr int C = kRowMaxK / 16 / kNqThreads;
+  if (M == 1) KRQ_NQ(kNqThreads, C, 1, true);
+  else if (K <= 4096) KRQ_NQ(256, 1, 4, false);
+  else KRQ_NQ(kNqThreads, C, kRowMaxK / 16 / 64, false);
+#undef KRQ_NQ
 }
 
 #define KRQ_FUSED_FP8_ARGS xb, x_scale, x_inv, x_per_row, wb, w_scale, w_per_row, m, NO, K, kts, out, nullptr, fa

@@ -243,6 +243,36 @@ KRQ_DEV uint2 quant8_clamped(uint4 v, float s) {
   return r;
 }
 
+KRQ_DEV bool finite_f32(float f) { return (as_u32(f) & 0x7f800000u) != 0x7f800000u; }
+
+// 16 bf16 times a finite inverse scale -> the 16 e4m3 bytes of quant8. CLAMPED: the products may exceed
+// 448. quant8 spends some twelve operations per value on the clamp that keeps NaN and the sign of a
+// NaN code; a piece without NaN or infinity (one packed maximum tells) needs neither.
+template <bool CLAMPED>
+KRQ_DEV uint4 quant16(uint4 a, uint4 b, float s) {
+  if (CLAMPED && bits_max_to_u32(absmax8_bits(b, absmax8_bits(a, u16x2{0, 0}))) >= 0x7f800000u) {
+    const uint2 lo = quant8(a, s), hi = quant8(b, s);
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+  }
+  const uint32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  uint32_t o[4];
+  auto q = [&](float f) { return CLAMPED ? __builtin_amdgcn_fmed3f(f * s, -kFp8Max, kFp8Max) : f * s; };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int p = __builtin_amdgcn_cvt_pk_fp8_f32(q(as_f32(v[2 * i] << 16)), q(as_f32(v[2 * i] & 0xffff0000u)), 0, false);
+    o[i] = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(q(as_f32(v[2 * i + 1] << 16)),
+                                                                 q(as_f32(v[2 * i + 1] & 0xffff0000u)), p, true));
+  }
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// 16 bf16 of a row times the inverse of the row's own amax a (NaN codes keep their signs)
+KRQ_DEV uint4 quant16_own_amax(uint4 v0, uint4 v1, float a, float inv) {
+  if (finite_f32(a)) return quant16<false>(v0, v1, inv);
+  const uint2 lo = quant8(v0, inv), hi = quant8(v1, inv);
+  return make_uint4(lo.x, lo.y, hi.x, hi.y);
+}
+
 // vector-ALU dot products (M == 1 kernels)
 KRQ_DEV float dot4_fp8(uint32_t a, uint32_t b, float acc) {
   const auto a0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)a, false);

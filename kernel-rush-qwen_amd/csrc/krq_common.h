@@ -143,9 +143,26 @@ KRQ_DEV uint32_t wave_max_u32_dpp(uint32_t v) {
   return umax32(umax32(r0, r1), umax32(r2, r3));
 }
 
+template <int CTRL>
+KRQ_DEV float dpp_f32(float v) {
+  return as_f32(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(as_u32(v)), CTRL, 0xf, 0xf, false)));
+}
+
+// Sum over the wave; every lane gets it (every lane active). The butterfly over lane distances 32, 16,
+// 8, 4, 2, 1, in that order: half and row swaps (v_permlane32_swap, v_permlane16_swap of a value with
+// itself give both halves' values), then DPP moves, a few cycles per step where a shuffle takes a
+// round trip through the LDS crossbar. The sums are the shuffles' bit for bit (an addition per step of
+// the same two values).
 KRQ_DEV float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 h = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);
+  v = as_f32(h[0]) + as_f32(h[1]);
+  const u32x2 q = __builtin_amdgcn_permlane16_swap(as_u32(v), as_u32(v), false, false);
+  v = as_f32(q[0]) + as_f32(q[1]);
+  v += dpp_f32<0x128>(v);                 // row_ror:8: lane ^ 8
+  v += dpp_f32<0x141>(dpp_f32<0x1B>(v));  // each quad reversed, then row_half_mirror: lane ^ 4
+  v += dpp_f32<0x4E>(v);                  // quad_perm(2,3,0,1): lane ^ 2
+  v += dpp_f32<0xB1>(v);                  // quad_perm(1,0,3,2): lane ^ 1
   return v;
 }
 

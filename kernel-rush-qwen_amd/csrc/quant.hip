@@ -417,11 +417,12 @@ __global__ __launch_bounds__(kQT) void k_act_rows_vec(const uint16_t* __restrict
   }
 }
 
-// quant_rows (K % 16 == 0): 16 values per thread piece (two 16-byte loads, one 16-byte store), the
-// row amax as DPP wave maxima and one barrier, 512 threads, one block per row. Measured on MI355X
-// (graph of 72 launches, M = 16; K = 2,560 / 4,096 / 9,728): 2.47 / 2.54 / 3.11 us against 2.87 /
-// 2.90 / 3.64 for k_act_rows_vec (256 threads, 8-value pieces, shuffle reductions, two barriers);
-// 256 and 1,024 threads measured slower.
+// quant_rows above 32 rows (K % 16 == 0): 16 values per thread piece (two 16-byte loads, one 16-byte
+// store), the row amax as DPP wave maxima and one barrier, 512 threads, one block per row, so the row
+// is read once (k_act_rows_wg reads it once per group of slices; few rows leave room for that).
+// Measured on MI355X (graph of 72 launches, M = 16; K = 2,560 / 4,096 / 9,728): 2.47 / 2.54 / 3.11 us
+// against 2.87 / 2.90 / 3.64 for k_act_rows_vec (256 threads, 8-value pieces, shuffle reductions, two
+// barriers); 256 and 1,024 threads measured slower.
 constexpr int kRowNT = 512;
 template <int NT>
 __global__ __launch_bounds__(NT) void k_act_rows_fast(const uint16_t* __restrict__ x, int64_t M, int64_t K,
@@ -452,14 +453,13 @@ __global__ __launch_bounds__(NT) void k_act_rows_fast(const uint16_t* __restrict
   for (int c = 0; c < C; ++c) {
     const int64_t e = 16 * (int64_t)(threadIdx.x + c * NT);
     if (e < K) {
-      const uint2 lo = quant8(v[c][0], iv), hi = quant8(v[c][1], iv);
-      *reinterpret_cast<uint4*>(x8 + r * K + e) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      *reinterpret_cast<uint4*>(x8 + r * K + e) = quant16_own_amax(v[c][0], v[c][1], a, iv);
     }
   }
 }
 
-// quant_rows_tiled by four-wave workgroups: workgroup (r, g) reads row r whole, wave w taking the
-// pieces of slices w + 4 c (c < CW; piece p = lane + 64 (w + 4 c), two 16-byte loads each, every
+// quant_rows up to 32 rows and quant_rows_tiled (TILED), by four-wave workgroups: workgroup (r, g)
+// reads row r whole, wave w taking the pieces of slices w + 4 c (c < CW; piece p = lane + 64 (w + 4 c), two 16-byte loads each, every
 // load in flight; pieces past the row repeat its last piece), so each lane loads 2 CW chunks instead
 // of the whole row's 2 ch. The waves' maxima (DPP within a wave) meet in LDS at one barrier; then
 // wave w quantizes slice w + 4 g, which it holds as its chunk c = g, into the tiled layout. Pad rows
@@ -469,8 +469,11 @@ __global__ __launch_bounds__(NT) void k_act_rows_fast(const uint16_t* __restrict
 // against 2.38 / 2.49 / 2.89 for single-wave workgroups that each read the whole row (one
 // workgroup per slice), 2.47 / 2.54 / 3.09 for one 512-thread block per row, and 3.21 / 3.69 /
 // 6.60 for one single-wave workgroup per row; eight-wave workgroups (two chunks per lane at
-// K = 9,728) measured 2.95 there.
-template <int CW>
+// K = 9,728) measured 2.95 there. The kernel is a chain: arguments, row, maximum, convert, store.
+// Without the NaN-keeping clamp in the convert (quant16_own_amax: some 190 instructions of a single
+// wave fewer) the decode step over eight layers takes 289.2 instead of 297.3 us at M = 16, and at
+// M = 5, where quant_rows moved here from 512-thread blocks as well, 277.2 instead of 290.4.
+template <int CW, bool TILED>
 __global__ __launch_bounds__(256) void k_act_rows_wg(const uint16_t* __restrict__ x, int64_t M, int64_t K,
                                                      float* __restrict__ scale, uint8_t* __restrict__ x8) {
   __shared__ uint32_t wmax[4];
@@ -478,7 +481,7 @@ __global__ __launch_bounds__(256) void k_act_rows_wg(const uint16_t* __restrict_
   const int64_t r = blockIdx.x;
   const int np = static_cast<int>(K >> 4);
   const int ps = lane + 64 * (w + 4 * gi);  // the piece this lane stores
-  if (r >= M) {  // (uniform per workgroup: no barrier below is skipped by part of it)
+  if (TILED && r >= M) {  // (uniform per workgroup: no barrier below is skipped by part of it)
     if (ps < np) *reinterpret_cast<uint4*>(x8 + tiled_offset(r, 16 * (int64_t)ps, K)) = zero4();
     return;
   }
@@ -504,8 +507,8 @@ __global__ __launch_bounds__(256) void k_act_rows_wg(const uint16_t* __restrict_
 #pragma unroll
     for (int c = 0; c < CW; ++c)
       if (c == gi) {
-        const uint2 lo = quant8(v[c][0], iv), hi = quant8(v[c][1], iv);
-        *reinterpret_cast<uint4*>(x8 + tiled_offset(r, 16 * (int64_t)ps, K)) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        const int64_t o = TILED ? tiled_offset(r, 16 * (int64_t)ps, K) : r * K + 16 * (int64_t)ps;
+        *reinterpret_cast<uint4*>(x8 + o) = quant16_own_amax(v[c][0], v[c][1], a, iv);
       }
   }
 }
@@ -521,27 +524,26 @@ __global__ __launch_bounds__(kQT) void k_cast_vec(const uint16_t* __restrict__ x
   }
 }
 
-KRQ_DEV bool finite_f32(float f) { return (as_u32(f) & 0x7f800000u) != 0x7f800000u; }
-
-// 16 bf16 times a finite inverse scale -> the 16 e4m3 bytes of quant8. CLAMPED: the products may exceed
-// 448. quant8 spends some twelve operations per value on the clamp that keeps NaN and the sign of a
-// NaN code; a piece without NaN or infinity (one packed maximum tells) needs neither.
-template <bool CLAMPED>
-KRQ_DEV uint4 quant16(uint4 a, uint4 b, float s) {
-  if (CLAMPED && bits_max_to_u32(absmax8_bits(b, absmax8_bits(a, u16x2{0, 0}))) >= 0x7f800000u) {
-    const uint2 lo = quant8(a, s), hi = quant8(b, s);
-    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+// the cast with a given inverse (krq_cast_fp8's bytes) into the tiled activation layout of
+// quant_rows_tiled: the M rows padded to a multiple of 16, one 16-value piece per thread, every load
+// of a row in flight at once, the pad rows written as zeros
+__global__ __launch_bounds__(kQT) void k_cast_rows_tiled(const uint16_t* __restrict__ x, int64_t M, int64_t K,
+                                                         const float* __restrict__ inv, uint8_t* __restrict__ x8) {
+  const int64_t r = blockIdx.x, p = blockIdx.y * (int64_t)kQT + threadIdx.x;
+  if (16 * p >= K) return;
+  uint4 o = zero4();
+  if (r < M) {
+    const uint8_t* src = reinterpret_cast<const uint8_t*>(x + r * K) + 32 * p;
+    const uint4 a = ld16(src), b = ld16(src + 16);
+    const float iv = inv[0];
+    if (finite_f32(iv)) {
+      o = quant16<true>(a, b, iv);
+    } else {
+      const uint2 lo = quant8(a, iv), hi = quant8(b, iv);
+      o = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    }
   }
-  const uint32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-  uint32_t o[4];
-  auto q = [&](float f) { return CLAMPED ? __builtin_amdgcn_fmed3f(f * s, -kFp8Max, kFp8Max) : f * s; };
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int p = __builtin_amdgcn_cvt_pk_fp8_f32(q(as_f32(v[2 * i] << 16)), q(as_f32(v[2 * i] & 0xffff0000u)), 0, false);
-    o[i] = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(q(as_f32(v[2 * i + 1] << 16)),
-                                                                 q(as_f32(v[2 * i + 1] & 0xffff0000u)), p, true));
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
+  *reinterpret_cast<uint4*>(x8 + tiled_offset(r, 16 * p, K)) = o;
 }
 
 // The cast's pieces of 16 values (np of them), two of a thread's at a time so that four 16-byte loads
@@ -574,28 +576,6 @@ KRQ_DEV void cast_pieces(const uint8_t* __restrict__ x, int64_t np, bool own, F 
     put(p + stride, a1, b1);
   }
   if (p < np) put(p, ld16(x + 32 * p), ld16(x + 32 * p + 16));
-}
-
-// the cast with a given inverse (krq_cast_fp8's bytes) into the tiled activation layout of
-// quant_rows_tiled: the M rows padded to a multiple of 16, one 16-value piece per thread, every load
-// of a row in flight at once, the pad rows written as zeros
-__global__ __launch_bounds__(kQT) void k_cast_rows_tiled(const uint16_t* __restrict__ x, int64_t M, int64_t K,
-                                                         const float* __restrict__ inv, uint8_t* __restrict__ x8) {
-  const int64_t r = blockIdx.x, p = blockIdx.y * (int64_t)kQT + threadIdx.x;
-  if (16 * p >= K) return;
-  uint4 o = zero4();
-  if (r < M) {
-    const uint8_t* src = reinterpret_cast<const uint8_t*>(x + r * K) + 32 * p;
-    const uint4 a = ld16(src), b = ld16(src + 16);
-    const float iv = inv[0];
-    if (finite_f32(iv)) {
-      o = quant16<true>(a, b, iv);
-    } else {
-      const uint2 lo = quant8(a, iv), hi = quant8(b, iv);
-      o = make_uint4(lo.x, lo.y, hi.x, hi.y);
-    }
-  }
-  *reinterpret_cast<uint4*>(x8 + tiled_offset(r, 16 * p, K)) = o;
 }
 
 // cast with given inverses (K % 16 == 0, so a piece lies in one row)
@@ -811,12 +791,29 @@ extern "C" int krq_cast_fp8(const void* x_bf16, int64_t M, int64_t K, const floa
   return krq_check_launch("cast_fp8");
 }
 
+// the four-wave workgroups over `rows` rows (M, or M padded to whole tiles); K % 16 == 0, K <= kVecMaxK
+template <bool TILED>
+static void launch_rows_wg(const void* x, int64_t M, int64_t K, int64_t rows, void* x8, float* xs, hipStream_t s) {
+  const int np = static_cast<int>(K / 16), ch = (np + 63) / 64;  // pieces per lane of a whole row (<= 16)
+  const int cw = (ch + 3) / 4;                                     // chunks per lane of a four-wave workgroup
+  const dim3 grid(static_cast<unsigned>(rows), static_cast<unsigned>(cw));
+#define KRQ_ROWS_WG(CW) \
+  hipLaunchKernelGGL((k_act_rows_wg<CW, TILED>), grid, dim3(256), 0, s, (const uint16_t*)x, M, K, xs, (uint8_t*)x8)
+  if (cw <= 1) KRQ_ROWS_WG(1);
+  else if (cw <= 2) KRQ_ROWS_WG(2);
+  else if (cw <= 3) KRQ_ROWS_WG(3);
+  else KRQ_ROWS_WG(4);
+#undef KRQ_ROWS_WG
+}
+
 extern "C" int krq_quant_rows(const void* x_bf16, int64_t M, int64_t K, void* x8, float* xs,
                               void* stream) {
   KRQ_REQUIRE(x_bf16 && x8 && xs, "quant_rows: null pointer");
   KRQ_REQUIRE(M > 0 && K > 0 && M <= 0x7fffffff, "quant_rows: bad shape M=%lld K=%lld",
               (long long)M, (long long)K);
-  if (vec_ok(x_bf16, K, K) && aligned16(x8) && K % 16 == 0)
+  if (vec_ok(x_bf16, K, K) && aligned16(x8) && K % 16 == 0 && M <= 32)
+    launch_rows_wg<false>(x_bf16, M, K, M, x8, xs, (hipStream_t)stream);
+  else if (vec_ok(x_bf16, K, K) && aligned16(x8) && K % 16 == 0)
     hipLaunchKernelGGL((k_act_rows_fast<kRowNT>), dim3(static_cast<unsigned>(M)), dim3(kRowNT), 0,
                        (hipStream_t)stream, (const uint16_t*)x_bf16, M, K, xs, (uint8_t*)x8);
   else if (vec_ok(x_bf16, K, K) && aligned16(x8))
@@ -836,17 +833,7 @@ extern "C" int krq_quant_rows_tiled(const void* x_bf16, int64_t M, int64_t K, vo
   KRQ_REQUIRE(vec_ok(x_bf16, K, K) && aligned16(x8_tiled),
               "quant_rows_tiled: x and x8_tiled must be 16-byte aligned and K at most %lld", (long long)kVecMaxK);
   const int64_t mp = (M + 15) / 16 * 16;  // rows padded to whole 16-row tiles
-  const int np = static_cast<int>(K / 16), ch = (np + 63) / 64;  // pieces per lane of a whole row (<= 16)
-  const int cw = (ch + 3) / 4;                                     // chunks per lane of a four-wave workgroup
-  const dim3 grid(static_cast<unsigned>(mp), static_cast<unsigned>(cw));
-#define KRQ_ROWS_WG(CW)                                                                                        \
-  hipLaunchKernelGGL((k_act_rows_wg<CW>), grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)x_bf16, M, K, \
-                     xs, (uint8_t*)x8_tiled)
-  if (cw <= 1) KRQ_ROWS_WG(1);
-  else if (cw <= 2) KRQ_ROWS_WG(2);
-  else if (cw <= 3) KRQ_ROWS_WG(3);
-  else KRQ_ROWS_WG(4);
-#undef KRQ_ROWS_WG
+  launch_rows_wg<true>(x_bf16, M, K, mp, x8_tiled, xs, (hipStream_t)stream);
   return krq_check_launch("quant_rows_tiled");
 }
 

@@ -147,6 +147,20 @@ def test_quant_rows(dev, M, K):
     assert np.array_equal(xs.cpu().numpy().reshape(-1), rs)
 
 
+# more than 32 rows (one block per row), and on either side of the line
+@pytest.mark.parametrize("M,K", [(32, 2560), (33, 2560), (33, 16384), (40, 80), (70, 9728)])
+def test_quant_rows_many(dev, M, K):
+    x = act(M, K, 8 + M)
+    x[M - 1] = 0.0
+    x[0, 0], x[1, 1], x[2, 2] = -0.0, float("nan"), float("inf")
+    x8, xs = fp8.quant_rows(x.to(dev))
+    xf = x.float()
+    amax = xf.abs().amax(1).clamp_min(1e-6)
+    r8 = (xf * (amax.reciprocal() * 448.0)[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn)
+    assert np.array_equal(xs.cpu().numpy().reshape(-1), O.div448(amax.numpy()), equal_nan=True)
+    assert np.array_equal(u8(x8), u8(r8))
+
+
 # ---------------------------------------------------------------------------------------------
 # weight quantizers and packing
 # ---------------------------------------------------------------------------------------------
