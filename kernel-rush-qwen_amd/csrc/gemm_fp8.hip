@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_fp8(const uint8_t* __restrict
 // bytes of row l % 32 of each operand fragment, k bytes 32 (l / 32) .. +31 of the 64-byte stage;
 // the product's element e of lane l belongs to first-operand row 8 (e / 4) + 4 (l / 32) + e % 4 and
 // second-operand row l % 32). K advances 64 bytes per stage; stages come in pairs whose 128 bytes
-// of each row fill one of two LDS pair buffers. Global bytes reach LDS with
+// of each row fill one of NB LDS pair buffers. Global bytes reach LDS with
 // global_load_lds_dwordx4: one instruction writes 1 KB, 8 rows of 128 bytes (whole lines), lane i
 // at byte 16 i, so a lane's global address picks which 16-byte chunk of which row lands at that
 // position. Chunk c of row r sits at position c ^ ((r >> 1) & 7) of its row: a ds_read_b128 serves
@@ -149,9 +149,9 @@ __global__ __launch_bounds__(kThreads) void k_gemm_fp8(const uint8_t* __restrict
 //
 // Per pair of stages (2j, 2j + 1): the even stage multiplies from registers and reads the odd
 // stage's fragments; the odd stage waits for the next pair's loads, passes a barrier (every wave's
-// loads have landed and every wave is done with pair j's buffer), issues the loads of pair j + 2
-// into that buffer, reads the next even stage's fragments and multiplies. Past the last stage the
-// loads go to a sink (one cached KB, same count).
+// loads have landed and every wave is done with pair j's buffer), issues the loads of pair j + NB
+// (NB pair buffers, two or four) into that buffer, reads the next even stage's fragments and
+// multiplies. Past the last stage the loads go to a sink (one cached KB, same count).
 namespace ring {
 
 constexpr int BK = 64, kThreads = 256;
@@ -210,14 +210,14 @@ struct StagePattern {
 // PART: each work unit is (tile, split): the tile's products over K / splits bytes of K, written
 // as fp32 to plane `split` of ws [splits][M][N] (k_splitk_reduce finishes them); otherwise one
 // unit per tile over all of K, written as bf16 with its scales applied.
-template <int BM, int BN, int OCC, bool PART>
+template <int BM, int BN, int OCC, bool PART, int NB = 2>
 __global__ __launch_bounds__(kThreads, OCC) void k_gemm_ring(const uint8_t* __restrict__ a, const float* __restrict__ asc,
                                                            int a_per_row, const uint8_t* __restrict__ b,
                                                            const float* __restrict__ bsc, int b_per_row, int M, int N,
                                                            int K, int tiles_m, int tiles, int splits, int ldo,
                                                            float* __restrict__ ws, uint16_t* __restrict__ out) {
   constexpr int kPairBytes = (BM + BN) * 2 * BK;  // two stages: 128 bytes of K per row, A rows then B rows
-  __shared__ __align__(1024) uint8_t ring[2 * kPairBytes];
+  __shared__ __align__(1024) uint8_t ring[NB * kPairBytes];
   __shared__ __align__(1024) float scl[2][BM + BN];  // per tile (alternating): row scales, then column scales
   __shared__ __align__(1024) uint8_t sink[1024];     // where the loads of stages past the last one land
   constexpr int FI = BM / 64, FJ = BN / 64;          // 32-row fragments of a wave's quarter
@@ -232,7 +232,8 @@ __global__ __launch_bounds__(kThreads, OCC) void k_gemm_ring(const uint8_t* __re
   constexpr int kStores = FI * 32 * CPR / 64;  // 16-byte stores per lane per tile
   constexpr int CR = kPairBytes >= 4 * 32 * RB ? 32 : 16;  // output rows per staging chunk
   static_assert((BM + BN) % 64 == 0, "scale loads");
-  static_assert(kVm + kStores < 64, "vmcnt range");
+  static_assert((NB - 1) * kVm + kStores < 64, "vmcnt range");
+  static_assert(NB >= 2 && (NB & (NB - 1)) == 0, "pair buffers: a power of two");
   static_assert(4 * CR * RB <= kPairBytes, "output staging fits one pair buffer");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int G = gridDim.x, bid = blockIdx.x;
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_gemm_ring(const uint8_t* __re
           0, 0, 0, 0);
       if (LOADS) {
 #pragma unroll
-        for (int l = u * NL / NP; l < (u + 1) * NL / NP; ++l) pair_load(l, (s + 3) / 2, pbl);
+        for (int l = u * NL / NP; l < (u + 1) * NL / NP; ++l) pair_load(l, s / 2 + NB, pbl);
       }
       if (READS) {
 #pragma unroll
@@ -427,9 +428,11 @@ __global__ __launch_bounds__(kThreads, OCC) void k_gemm_ring(const uint8_t* __re
     // branches around its store), so after such a tile the wait counts only the second pair.
     lds_barrier();
 #pragma unroll
-    for (int q = 0; q < kVm; ++q) pair_load(q, 1, 1);
-    if (k == 0 || ragged) wait_vm<kVm>();
-    else wait_vm<kVm + kStores>();
+    for (int j = 1; j < NB; ++j)
+#pragma unroll
+      for (int q = 0; q < kVm; ++q) pair_load(q, j, j);
+    if (k == 0 || ragged) wait_vm<(NB - 1) * kVm>();
+    else wait_vm<(NB - 1) * kVm + kStores>();
     lds_barrier();
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
@@ -445,13 +448,13 @@ __global__ __launch_bounds__(kThreads, OCC) void k_gemm_ring(const uint8_t* __re
     const int cm0 = m0, cn0 = n0, csp = sp;
     const int next = tile_of(k + 1);
     for (int s = 0; s < nk - 2; s += 2) {
-      const int pb = (s >> 1) & 1;
+      const int pb = (s >> 1) & (NB - 1);
       body(even{}, no{}, yes{}, s, pb, 0);
-      wait_vm<0>();  // the pair of stages s + 2, s + 3
+      wait_vm<(NB - 2) * kVm>();  // the pair of stages s + 2, s + 3
       lds_barrier();
-      body(odd{}, yes{}, yes{}, s + 1, pb ^ 1, pb);
+      body(odd{}, yes{}, yes{}, s + 1, (pb + 1) & (NB - 1), pb);
     }
-    body(even{}, no{}, yes{}, nk - 2, ((nk - 2) >> 1) & 1, 0);
+    body(even{}, no{}, yes{}, nk - 2, ((nk - 2) >> 1) & (NB - 1), 0);
     // last stage: once every wave is past this barrier the ring is free; the next tile starts loading
     lds_barrier();
     if (next >= 0) {
@@ -587,11 +590,11 @@ int gemm_run(const void* x, int x_kind, const float* x_scale, const float* x_inv
     if (rp.splits > 1 && (!aligned16(ws) || ws_bytes < (int64_t)rp.splits * M * N * 4)) rp.splits = 1;
     if (rp.bm > 0) {
       // one launch over columns [n_lo, n_hi) of the output (ldo = N)
-#define KRQ_RING(BM_, BN_, OCC_, PART_, n_lo, n_hi)                                                                  \
+#define KRQ_RING(BM_, BN_, OCC_, PART_, NB_, n_lo, n_hi)                                                                \
   do {                                                                                                             \
     const int64_t nn = (n_hi) - (n_lo), tm_ = (M + (BM_)-1) / (BM_), tiles_ = tm_ * (nn / (BN_));                   \
     const int64_t units_ = tiles_ * rp.splits, slots_ = (int64_t)cus * (OCC_);                                     \
-    hipLaunchKernelGGL((ring::k_gemm_ring<BM_, BN_, OCC_, PART_>), dim3(static_cast<unsigned>(units_ < slots_ ? units_ : slots_)), \
+    hipLaunchKernelGGL((ring::k_gemm_ring<BM_, BN_, OCC_, PART_, NB_>), dim3(static_cast<unsigned>(units_ < slots_ ? units_ : slots_)), \
                        dim3(ring::kThreads), 0, s, (const uint8_t*)x, x_scale, x_per_row,                           \
                        (const uint8_t*)w8 + (n_lo) * K, w_scale + (w_per_row ? (n_lo) : 0), w_per_row, (int)M,     \
                        (int)nn, (int)K, (int)tm_, (int)tiles_, rp.splits, (int)N, (float*)ws,                       \
@@ -601,28 +604,39 @@ int gemm_run(const void* x, int x_kind, const float* x_scale, const float* x_inv
         // the whole rounds' tiles (M-fastest) fill whole columns of tiles: the first n_split columns
         const int64_t tm256 = (M + 255) / 256, rounds = (N / 256) * tm256 / cus;
         const int64_t n_split = rounds * cus / tm256 * 256;
-        KRQ_RING(256, 256, 1, false, 0, n_split);
-        KRQ_RING(128, 128, 2, false, n_split, N);
+        KRQ_RING(256, 256, 1, false, 2, 0, n_split);
+        KRQ_RING(128, 128, 2, false, 2, n_split, N);
       } else if (rp.bm == 256) {
-        KRQ_RING(256, 256, 1, false, 0, N);
+        KRQ_RING(256, 256, 1, false, 2, 0, N);
       } else if (rp.bm == 192) {
-        KRQ_RING(192, 256, 1, false, 0, N);
-      } else if (rp.bm == 64 && rp.splits == 1) {
-        KRQ_RING(64, 64, 4, false, 0, N);
-      } else if (rp.bm == 64) {
-        KRQ_RING(64, 64, 4, true, 0, N);
-        const int64_t threads = M * N / 4;
-        hipLaunchKernelGGL(ring::k_splitk_reduce, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s,
-                           (const float*)ws, rp.splits, (int)M, (int)N, x_scale, x_per_row, w_scale, w_per_row,
-                           (uint16_t*)out);
-      } else if (rp.splits == 1) {
-        KRQ_RING(128, 128, 2, false, 0, N);
+        KRQ_RING(192, 256, 1, false, 2, 0, N);
       } else {
-        KRQ_RING(128, 128, 2, true, 0, N);
-        const int64_t threads = M * N / 4;
-        hipLaunchKernelGGL(ring::k_splitk_reduce, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s,
-                           (const float*)ws, rp.splits, (int)M, (int)N, x_scale, x_per_row, w_scale, w_per_row,
-                           (uint16_t*)out);
+        const int64_t units = (M + rp.bm - 1) / rp.bm * (N / rp.bm) * rp.splits;
+        // Four pair buffers where the grid leaves LDS for them (at most one workgroup of 128 x 128
+        // tiles or two of 64 x 64 per compute unit): a workgroup alone on its unit waits for one
+        // pair's latency per pair with two. Weights cold in the caches, two -> four buffers, us: M =
+        // 64 QKV 11.1 -> 7.2, O 15.8 -> 9.4, down 14.2 -> 10.7; M = 256 O 15.8 -> 9.6, down 20.0 ->
+        // 17.0; eight buffers (one workgroup per unit) measured 7.9, 9.3 and 11.1 at M = 64.
+        const bool deep = units <= (rp.bm == 64 ? 2 : 1) * (int64_t)cus;
+#define KRQ_RING_DEEP(BM_, OCC_, PART_)                            \
+  if (deep) KRQ_RING(BM_, BM_, OCC_ / 2, PART_, 4, 0, N);          \
+  else KRQ_RING(BM_, BM_, OCC_, PART_, 2, 0, N)
+        if (rp.bm == 64 && rp.splits == 1) {
+          KRQ_RING_DEEP(64, 4, false);
+        } else if (rp.bm == 64) {
+          KRQ_RING_DEEP(64, 4, true);
+        } else if (rp.splits == 1) {
+          KRQ_RING_DEEP(128, 2, false);
+        } else {
+          KRQ_RING_DEEP(128, 2, true);
+        }
+#undef KRQ_RING_DEEP
+        if (rp.splits > 1) {
+          const int64_t threads = M * N / 4;
+          hipLaunchKernelGGL(ring::k_splitk_reduce, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s,
+                             (const float*)ws, rp.splits, (int)M, (int)N, x_scale, x_per_row, w_scale, w_per_row,
+                             (uint16_t*)out);
+        }
       }
 #undef KRQ_RING
       return krq_check_launch("gemm_fp8");

@@ -27,9 +27,13 @@ from . import _lib as L
 FP8_MAX = 448.0
 HEADROOM = float(os.environ.get("ENGINE_FP8_HEADROOM", "4"))
 DECODE_MAX_ROWS = 32  # rows handled by one launch of the skinny kernels
-# From this many rows linear_fp8 runs gemm_fp8: per Qwen3-4B decoder layer (the four projections)
-# it takes 0.80x-0.995x hipBLASLt's time on MI355X from M = 128 to 4096, and 1.09x at M = 64.
-PREFILL_MIN_ROWS = 128
+# From this many rows linear_fp8 runs gemm_fp8. Per Qwen3-4B decoder layer (the four projections,
+# weights cold in the caches) against hipBLASLt on MI355X, us: M = 33 39.2 / 39.5, M = 48 40.0 / 43.3,
+# M = 77 44.2 / 46.9, M = 127 46.8 / 51.8, M = 160 54.8 / 54.4, M = 256 58.1 / 67.4, M = 1024 133 / 141;
+# and the library's call takes 20 us of host time where this one takes 8.
+PREFILL_MIN_ROWS = DECODE_MAX_ROWS + 1
+# The library takes one scale per weight; fewer rows than this keep refusing per-channel ones there.
+PER_CHANNEL_MIN_ROWS = 128
 
 
 class FP8Weight(tuple):
@@ -463,10 +467,10 @@ def gemm_fp8(x, q, a=None, xs=None):
 def linear_fp8(x, q, a=None, amax_out=None):
     """bf16 [M, N] ~= x @ W^T with q = quantize_weight(W); a = given scale, or
     None to scale by this tensor's own range (running max kept in amax_out).
-    Reference: engine/kernels/fp8.py:97-106. Decode sizes (M <= 32) run the HIP GEMV; prefill
-    rows from PREFILL_MIN_ROWS up run this library's GEMM (gemm_fp8) where its e4m3 kernels take
-    the weight (N and K multiples of 128, K >= 256); the rest keep the reference's library GEMM,
-    torch._scaled_mm (hipBLASLt on ROCm)."""
+    Reference: engine/kernels/fp8.py:97-106. Decode sizes (M <= 32) run the HIP GEMV; more rows
+    run this library's GEMM (gemm_fp8) where its e4m3 kernels take the weight (N and K multiples of
+    128, K >= 256); the rest keep the reference's library GEMM, torch._scaled_mm (hipBLASLt on
+    ROCm)."""
     w8, ws = q[0], q[1]
     x8 = None
     if a is None:
@@ -484,7 +488,7 @@ def linear_fp8(x, q, a=None, amax_out=None):
         x8 = _cast(x, a)
     if x.shape[0] <= DECODE_MAX_ROWS:
         return gemv_fp8_launch(x8, a.scale.reshape(1), q, 1, L.OUT_BF16)
-    if x.shape[0] >= PREFILL_MIN_ROWS and _ring_gemm_fits(w8):
+    if x.shape[0] >= (PREFILL_MIN_ROWS if ws.numel() == 1 else PER_CHANNEL_MIN_ROWS) and _ring_gemm_fits(w8):
         return gemm_fp8(x8, q, xs=a.scale.reshape(1))
     return torch._scaled_mm(x8, w8.t(), scale_a=a.scale, scale_b=ws, out_dtype=torch.bfloat16)
 

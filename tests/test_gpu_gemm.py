@@ -156,6 +156,36 @@ def test_linear_fp8_prefill_route(dev, M, N, K):
     assert rel_err(y.float().cpu().numpy(), ref) <= TOL
 
 
+# Four pair buffers: fewer pairs of stages than buffers (K = 256, 384), as many, one more; rows from
+# the first the GEMM takes, ragged and whole tiles; two 64 x 64 units per compute unit and one tile
+# more (N = 16,512: two buffers); 128 x 128 tiles, split K on either kind, one part per unit or past it.
+@pytest.mark.parametrize("M,N,K", [(33, 128, 256), (64, 128, 384), (77, 256, 512), (65, 384, 640), (127, 128, 1152),
+                                   (100, 16384, 256), (100, 16512, 256), (33, 2560, 9728), (127, 2560, 9728),
+                                   (129, 2560, 9728), (300, 2560, 8192), (200, 2560, 4096)])
+def test_gemm_deep_ring(dev, M, N, K):
+    q = F.quantize(bf((N, K), 51, 0.02).to(dev))
+    for seed in (52, 53):  # (the second over the first's leftovers in LDS and the workspace)
+        x8, xs = F.quant_rows(bf((M, K), seed).to(dev))
+        y = F.gemm_fp8(x8, q, xs=xs)
+        ref = (x8.double() @ q[0].double().t()) * xs.double() * q[1].double()
+        assert rel_err(y.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
+        assert torch.equal(F.gemm_fp8(x8, q, xs=xs), y)
+
+
+@pytest.mark.parametrize("M,takes", [(33, False), (127, False), (128, True)])
+def test_linear_fp8_per_channel_rows(dev, M, takes):
+    """Per-channel weights: refused below 128 rows (the library's scaled product takes one scale per
+    weight), this library's GEMM from there."""
+    q = F.quantize(bf((256, 512), 54, 0.02).to(dev))
+    x = bf((M, 512), 55).to(dev)
+    if takes:
+        a = F.ActScale(x)
+        assert torch.equal(F.linear_fp8(x, q), F.gemm_fp8(F._cast(x, a), q, xs=a.scale.reshape(1)))
+    else:
+        with pytest.raises((RuntimeError, ValueError)):
+            F.linear_fp8(x, q)
+
+
 @pytest.mark.parametrize("M,N,K", [(4096, 6144, 512), (256, 2560, 9728), (300, 6144, 2560)])
 def test_gemm_graph_replays(dev, M, N, K):
     """gemm_fp8 captured in a graph (the two-launch tail plan, split K with its reduce and the
