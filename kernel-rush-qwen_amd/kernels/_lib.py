@@ -103,11 +103,14 @@ def call(name, *args):
 
 
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """The device address, as the integer ctypes takes for a void* argument."""
+    return None if t is None else t.data_ptr()
 
 
 def stream(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """torch's current stream on t's device, as its raw handle: torch.cuda.current_stream(t.device)
+    .cuda_stream without the Stream object (0.1 instead of 2.1 us of a call that launches in 3.6)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def require_device(*tensors):

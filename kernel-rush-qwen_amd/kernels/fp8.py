@@ -159,7 +159,7 @@ def cast_tiled(x, a):
     L.require_device(a.inv)
     mp = (M + 15) // 16 * 16
     x8t = torch.empty((mp * K,), device=x2.device, dtype=torch.uint8)
-    L.call("krq_cast_fp8_tiled", L.ptr(x2), M, K, L.ptr(a.inv.reshape(1)), L.ptr(x8t), L.stream(x2))
+    L.call("krq_cast_fp8_tiled", L.ptr(x2), M, K, L.ptr(_one(a.inv)), L.ptr(x8t), L.stream(x2))
     return x8t
 
 
@@ -296,7 +296,12 @@ def gemv_fp8_bf16_launch(x, q, split=1, mode=L.OUT_BF16, a=None, algo=L.ALGO_AUT
     M = x.shape[0]
     if a is None:
         return _gemv(x, L.X_BF16_DYN, None, None, M, q, split, mode, algo, out)
-    return _gemv(x, L.X_BF16_STATIC, a.scale.reshape(1), a.inv.reshape(1), M, q, split, mode, algo, out)
+    return _gemv(x, L.X_BF16_STATIC, _one(a.scale), _one(a.inv), M, q, split, mode, algo, out)
+
+
+def _one(scale):
+    """A per-tensor scale as the launches take it: one value (0-d or [1])."""
+    return scale if scale.numel() == 1 else scale.reshape(1)
 
 
 def _fits_fused(x, split, a):
@@ -321,7 +326,7 @@ def _activation_fp8(x, a, xs):
             raise ValueError("float8 activations need their scale xs")
         return x.contiguous(), xs.reshape(-1).contiguous()
     if a is not None:
-        return _cast(x, a), a.scale.reshape(1)
+        return _cast(x, a), _one(a.scale)
     x8, s = quant_rows(x)
     return x8, s.reshape(-1)
 
@@ -348,7 +353,7 @@ def _tiled_operand(x, a):
     """(x8 tiled, x_scale) for _tiled_rows inputs: per token, or with the given scale."""
     if a is None:
         return quant_rows_tiled(x)
-    return cast_tiled(x, a), a.scale.reshape(1)
+    return cast_tiled(x, a), _one(a.scale)
 
 
 def _chunked(x8, xs, fn):
@@ -410,7 +415,7 @@ def swiglu_cast_fp8(x, q, out_a, a=None, xs=None):
     if xs is None and _fits_fused(x, 1, a):
         xin = _rows(x)
         kind, x_scale, x_inv = (L.X_BF16_DYN, None, None) if a is None else \
-            (L.X_BF16_STATIC, a.scale.reshape(1), a.inv.reshape(1))
+            (L.X_BF16_STATIC, _one(a.scale), _one(a.inv))
     elif _tiled_rows(x, a, xs, L.ALGO_AUTO):
         xin, x_scale = _tiled_operand(x, a)
         kind, x_inv = L.X_FP8_TILED, None
@@ -450,8 +455,8 @@ def gemm_fp8(x, q, a=None, xs=None):
         if a is None:
             raise ValueError("bf16 activations need an ActScale / SharedScale a")
         if K % 128 == 0 and K >= 256:
-            return gemm_fp8(_cast_hip(_rows(x), a), q, xs=a.scale.reshape(1))
-        kind, xin, x_scale, x_inv = L.X_BF16_STATIC, _rows(x), a.scale.reshape(1), a.inv.reshape(1)
+            return gemm_fp8(_cast_hip(_rows(x), a), q, xs=_one(a.scale))
+        kind, xin, x_scale, x_inv = L.X_BF16_STATIC, _rows(x), _one(a.scale), _one(a.inv)
     L.require_device(x_scale, x_inv)
     xpr = 1 if (x_scale.numel() == M and M > 1) else 0
     out = torch.empty((M, N), device=x.device, dtype=torch.bfloat16)
@@ -472,6 +477,9 @@ def linear_fp8(x, q, a=None, amax_out=None):
     128, K >= 256); the rest keep the reference's library GEMM, torch._scaled_mm (hipBLASLt on
     ROCm)."""
     w8, ws = q[0], q[1]
+    if (x.dim() == 2 and _cast is _cast_hip and _ring_gemm_fits(w8)
+            and x.shape[0] >= (PREFILL_MIN_ROWS if ws.numel() == 1 else PER_CHANNEL_MIN_ROWS)):
+        return _linear_gemm(x, q, a, amax_out)
     x8 = None
     if a is None:
         if x.dim() == 2 and x.shape[0] > DECODE_MAX_ROWS and _cast is _cast_hip:
@@ -483,14 +491,51 @@ def linear_fp8(x, q, a=None, amax_out=None):
     if x8 is None and _fits_fused(x, 1, a):
         return gemv_fp8_bf16_launch(x, q, 1, L.OUT_BF16, a)
     if x8 is None and _tiled_rows(x, a, None, L.ALGO_AUTO):
-        return gemv_fp8_tiled_launch(cast_tiled(x, a), a.scale.reshape(1), q, x.shape[0], 1, L.OUT_BF16)
+        return gemv_fp8_tiled_launch(cast_tiled(x, a), _one(a.scale), q, x.shape[0], 1, L.OUT_BF16)
     if x8 is None:
         x8 = _cast(x, a)
     if x.shape[0] <= DECODE_MAX_ROWS:
-        return gemv_fp8_launch(x8, a.scale.reshape(1), q, 1, L.OUT_BF16)
+        return gemv_fp8_launch(x8, _one(a.scale), q, 1, L.OUT_BF16)
     if x.shape[0] >= (PREFILL_MIN_ROWS if ws.numel() == 1 else PER_CHANNEL_MIN_ROWS) and _ring_gemm_fits(w8):
-        return gemm_fp8(x8, q, xs=a.scale.reshape(1))
+        return gemm_fp8(x8, q, xs=_one(a.scale))
     return torch._scaled_mm(x8, w8.t(), scale_a=a.scale, scale_b=ws, out_dtype=torch.bfloat16)
+
+
+def _linear_gemm(x, q, a, amax_out):
+    """linear_fp8 on the ring GEMM: the scale (without a given one), the cast and the product, their
+    scale, e4m3 rows and partials in one allocation beside the output. A call on a short prompt is
+    host work (the launches take 3 us each): 37 us with an allocation per piece and the launches
+    through ActScale and gemm_fp8, 20 us this way."""
+    w8, ws = q[0], q[1]
+    N, K = w8.shape
+    x2 = _rows(x)
+    M = x2.shape[0]
+    L.require_device(w8, ws)
+    if x2.shape[1] != K:
+        raise ValueError(f"x {tuple(x.shape)} does not match w8 {tuple(w8.shape)}")
+    lib = L.lib()
+    parts = 4 * lib.krq_act_scale_ws_floats(M, K) if a is None else 0
+    split_bytes = lib.krq_gemm_fp8_ws_bytes(L.X_FP8, M, N, K)
+    if split_bytes < 0:
+        raise RuntimeError("krq_gemm_fp8_ws_bytes: device query failed")
+    # amax, inv, scale and the maxima's partials | e4m3 rows | split-K partials
+    at8 = (16 + parts + 255) & -256
+    at_split = (at8 + M * K + 255) & -256
+    work = torch.empty(at_split + split_bytes, device=x2.device, dtype=torch.uint8)
+    out = torch.empty((M, N), device=x2.device, dtype=torch.bfloat16)
+    p, st = work.data_ptr(), L.stream(x2)
+    if a is None:
+        scale = p + 8
+        L.call("krq_act_scale_cast_fp8", L.ptr(x2), M, K, 1.0, p, p + 4, scale, p + 16, p + at8, st)
+        if amax_out is not None:
+            amax_out.copy_(torch.maximum(amax_out, work[:4].view(torch.float32)))
+    else:
+        L.require_device(a.inv, a.scale)
+        scale = L.ptr(_one(a.scale))
+        L.call("krq_cast_fp8", L.ptr(x2), M, K, L.ptr(a.inv), 0, p + at8, st)
+    L.call("krq_gemm_fp8_ws", p + at8, L.X_FP8, scale, None, 0, L.ptr(w8), L.ptr(ws), 1 if ws.numel() > 1 else 0,
+           M, N, K, p + at_split if split_bytes else None, split_bytes, L.ptr(out), st)
+    return out
 
 
 def _ring_gemm_fits(w8):
