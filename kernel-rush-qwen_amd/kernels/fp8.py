@@ -337,15 +337,22 @@ def _activation_fp8(x, a, xs):
 # 7.52 / 7.40; gate_up M = 4 12.64 / 13.47, M = 16 14.19 / 13.70; down M = 4 9.70 / 10.35, M = 16
 # 11.24 / 10.83; given scale M = 8 QKV 7.19 / 7.60, M = 16 8.25 / 7.68, M = 32 10.47 / 9.29.
 TILED_MIN_ROWS = 13
+# Split-K GEMVs take the tiled rows earlier: their workgroups share them in LDS (k_gemv_wide32), where
+# one K pass over a whole row measures slower on them below 13 rows (linear_fp8 over a layer's four
+# projections at M = 5 36.4 us row-major, 43.0 tiled). With a given scale from three rows, scaled per
+# token from ten (QKV, O, gate_up and down of eight layers in one graph, row-major / tiled, us: given
+# M = 2 273.8 / 279.7, M = 3 291.5 / 282.4, M = 7 303.7 / 288.2; per token M = 9 284.8 / 287.1, M = 10
+# 299.2 / 298.0, M = 12 305.2 / 298.7).
+TILED_MIN_ROWS_SPLIT = {"given": 3, "token": 11}
 
 
-def _tiled_rows(x, a, xs, algo):
-    """bf16 rows at TILED_MIN_ROWS <= M <= 32 go through quant_rows_tiled (scaled per token) or
+def _tiled_rows(x, a, xs, algo, least=TILED_MIN_ROWS):
+    """bf16 rows at `least` <= M <= 32 go through quant_rows_tiled (scaled per token) or
     cast_tiled (a given scale) and the GEMV on tiled activations (the operands of quant_rows / _cast
     + the row-major e4m3 GEMV, with contiguous loads); fewer rows, and rows longer than the tiled
     kernels take, use the row-major kernels."""
     M, K = x.shape
-    return (xs is None and x.dtype == torch.bfloat16 and TILED_MIN_ROWS <= M <= DECODE_MAX_ROWS
+    return (xs is None and x.dtype == torch.bfloat16 and least <= M <= DECODE_MAX_ROWS
             and K % 64 == 0 and K <= TILED_ROWS_MAX_K and algo != L.ALGO_VALU)
 
 
@@ -378,7 +385,8 @@ def gemv_fp8(x, q, split=1, a=None, xs=None, algo=L.ALGO_AUTO):
     mode = L.OUT_BF16 if split == 1 else L.OUT_PARTIAL
     if xs is None and _fits_fused(x, split, a):
         return gemv_fp8_bf16_launch(x, q, split, mode, a, algo)
-    if _tiled_rows(x, a, xs, algo):
+    least = TILED_MIN_ROWS if split == 1 else TILED_MIN_ROWS_SPLIT["token" if a is None else "given"]
+    if _tiled_rows(x, a, xs, algo, least):
         x8t, s = _tiled_operand(x, a)
         return gemv_fp8_tiled_launch(x8t, s, q, M, split, mode)
     x8, s = _activation_fp8(x, a, xs)

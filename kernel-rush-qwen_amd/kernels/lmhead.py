@@ -6,7 +6,7 @@ reference's fused form keeps the same rule (engine/kernels/mega.py:412-436).
 
 FP8 heads take the activation scaling of the weight's form:
   per-channel weights (fp8.quantize, BASELINE's per-channel lm_head): h scaled per token, inside
-      the GEMV at M == 1, else by fp8.quant_rows (row-major rows) or, from fp8.TILED_MIN_ROWS,
+      the GEMV at M == 1, else by fp8.quant_rows (row-major rows) or, from TILED_MIN_ROWS,
       fp8.quant_rows_tiled (rows in the tiled activation layout);
   per-tensor weights (fp8.quantize_weight, the engine's lm8 = quantize_weight(lm_head),
       engine.py:504-505): exactly linear_fp8(h, lm8) followed by torch.argmax (engine.py:989,
@@ -19,6 +19,12 @@ import torch
 from . import _lib as L
 from . import fp8 as _fp8
 from . import gemv as _gemv
+
+
+# The persistent head reads tiled rows from LDS (k_lmhead_fp8_persist); fewer rows cost less row-major,
+# without the padding to sixteen. Measured at V = 151,936, ids and logits, us row-major / tiled: M = 2
+# 73.7 / 75.5, M = 4 64.8 / 68.1, M = 5 70.5 / 68.5, M = 6 71.1 / 68.0, M = 12 78.5 / 69.5.
+TILED_MIN_ROWS = 5
 
 
 def _fp8_operands(h, w, a, h_layout):
@@ -36,7 +42,7 @@ def _fp8_operands(h, w, a, h_layout):
     if ws.numel() == 1:          # linear_fp8's own ActScale over the whole of h
         a = _fp8.ActScale(h)
         return _fp8._cast(_fp8._rows(h), a), a.scale.reshape(1), 0, L.LM_FP8
-    tiled = h_layout == "tiled" or (h_layout == "auto" and M >= _fp8.TILED_MIN_ROWS)
+    tiled = h_layout == "tiled" or (h_layout == "auto" and M >= TILED_MIN_ROWS)
     if K % 64 == 0 and K <= _fp8.TILED_ROWS_MAX_K and tiled:   # tiled e4m3 rows
         h8, hs = _fp8.quant_rows_tiled(h)
         return h8, hs.reshape(-1), 1, L.LM_FP8_TILED_H
@@ -49,9 +55,7 @@ def lm_head_argmax(h, w, return_logits=False, h_layout="auto", a=None):
     fp8.quantize (per channel) or fp8.quantize_weight (per tensor). Returns int64 [M] token ids,
     or (ids, bf16 logits [M, V]) with return_logits=True. h_layout ("auto", "tiled" or
     "rowmajor"): how a per-channel FP8 head's per-token rows are laid out at M > 1 (the same
-    operands either way); "auto" takes tiled rows from fp8.TILED_MIN_ROWS (measured on MI355X at
-    V = 151,936, us tiled / row-major: M = 2 68.4 / 63.8, M = 8 72.9 / 71.5, M = 12 75.5 / 75.4,
-    M = 16 77.5 / 80.7). a: an ActScale / SharedScale for the FP8 head's activations (as
+    operands either way); "auto" takes tiled rows from TILED_MIN_ROWS. a: an ActScale / SharedScale for the FP8 head's activations (as
     linear_fp8 takes), instead of the scaling described in the module docstring."""
     L.require_device(h)
     M, K = h.shape
