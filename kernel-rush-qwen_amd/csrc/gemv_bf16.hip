@@ -237,6 +237,146 @@ __global__ __launch_bounds__(512) void k_gemv_bf16(const uint8_t* __restrict__ x
   gemv_bf16_body<MT, MODE, LAYOUT, ALGO, U, PB, XO>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
 }
 
+// Wide blocks at 4 < M <= 32: a workgroup of four waves owns four adjacent row blocks (one per wave, 64
+// output columns; P = 2: of both halves of the SwiGLU) of one K split. A 16-column block brings as
+// many activation bytes from L2 as weight bytes at M = 16 (twice as many at M = 32); here the split's
+// activation rows go to LDS once for the four, by direct-to-LDS loads of whole lines, and each wave
+// streams only its weights through a ring of U step slots. Steps, products and sums are those of the
+// NS-wave launch it replaces: step j goes to accumulator set j % NS, the sets are added from zero in
+// wave order, so the results are the same bit for bit.
+// LDS: step j of row group h (rows 8 h .. 8 h + 7 of the HV in use) is 1 KiB at (j HV + h) KiB, entry
+// 8 (c ^ (h % 2)) + row the row's 16-byte chunk c: a wave's operand read (rows 0-7 of one group, 8-15 of
+// the next, one chunk) then covers 256 consecutive bytes modulo the banks.
+constexpr int kWideRb = 4;
+
+KRQ_DEV void wide_dma(const uint8_t* base, uint32_t voff, uint32_t l) {
+  // (waited for by hand: issued before every other load, and vector memory loads complete in order)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l), "v"(voff), "s"(base)
+               : "memory", "m0");
+}
+
+template <int MODE, int LAYOUT, int MT, int U, int NS, int TL>
+__global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* __restrict__ x,
+                                                                 const uint8_t* __restrict__ w, int M, int64_t NO,
+                                                                 int64_t K, int kts, void* __restrict__ out) {
+  constexpr int P = MODE == KRQ_OUT_SWIGLU ? 2 : 1;
+  constexpr bool RM = LAYOUT == KRQ_W_ROWMAJOR;
+  static_assert(U % NS == 0 && 2 * P * U < 64, "slot u feeds set u % NS; vmcnt range");
+  __shared__ __align__(1024) uint8_t xt[TL * 1024];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int r = lane & 15, g = lane >> 4;
+  const int sidx = blockIdx.y;
+  const int64_t rb = (int64_t)blockIdx.x * kWideRb + wave;
+  const int nsteps = (kts + 1) >> 1, hv = (M + 7) >> 3;
+  const int64_t tbase = (int64_t)sidx * kts, rowb = 2 * K;
+
+  const uint32_t lx = __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)xt)));
+  for (int i = wave; i < nsteps * hv; i += kWideRb) {
+    const int j = i / hv, h = i - j * hv;
+    int c = (lane >> 3) ^ (h & 1);
+    if (2 * j + 1 >= kts) c &= 3;  // (a half last step: the high chunks repeat the low ones, masked below)
+    wide_dma(x, static_cast<uint32_t>(min(8 * h + (lane & 7), M - 1) * rowb + (tbase + 2 * j) * 64 + 16 * c),
+             lx + 1024u * static_cast<uint32_t>(i));
+  }
+  uint4 wl[P][U], wh[P][U];
+  auto load_slot = [&](int u, int cc) {  // (a slot past the last step reloads it, masked where consumed)
+    const int j = min(cc, nsteps - 1);
+    const int64_t t0 = tbase + 2 * j, t1 = (2 * j + 1 < kts) ? t0 + 1 : t0;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int64_t rr = p == 1 ? rb + (NO >> 4) : rb;
+      if constexpr (RM) {
+        const uint8_t* a = w + (16 * rr + (r & 7)) * rowb + t0 * 64 + 16 * w_line_chunk(lane, 2 * j + 1 >= kts);
+        wl[p][u] = ld16nt(a);
+        wh[p][u] = ld16nt(a + 8 * rowb);
+      } else {
+        wl[p][u] = ld16nt(w_addr<LAYOUT>(w, rr, t0, rowb, lane));
+        wh[p][u] = ld16nt(w_addr<LAYOUT>(w, rr, t1, rowb, lane));
+      }
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    load_slot(u, u);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * P * U) : "memory");  // (the activation rows have landed)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+
+  v4f acc[P][NS][MT];
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+#pragma unroll
+    for (int q = 0; q < NS; ++q)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[p][q][mt] = v4f{0.f, 0.f, 0.f, 0.f};
+  auto consume = [&](int u, int cc) {
+    const int j = min(cc, nsteps - 1);
+    const bool ok = cc < nsteps, hi = ok && (2 * j + 1 < kts);
+    uint4 al[MT], ah[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {  // (rows past the groups in use read the last group)
+      const int h = min(2 * mt + (r >> 3), hv - 1);
+      const uint8_t* xr = xt + (j * hv + h) * 1024 + 16 * (r & 7);
+      al[mt] = *reinterpret_cast<const uint4*>(xr + 128 * (g ^ (h & 1)));
+      ah[mt] = *reinterpret_cast<const uint4*>(xr + 128 * ((g + 4) ^ (h & 1)));
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      uint4 bl = wl[p][u], bh = wh[p][u];
+      if constexpr (RM) lines_to_tiles(wl[p][u], wh[p][u], &bl, &bh);
+      bl = sel4(ok, bl);
+      bh = sel4(hi, bh);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        v4f& c = acc[p][u % NS][mt];
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_v8bf(al[mt]), as_v8bf(bl), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_v8bf(ah[mt]), as_v8bf(bh), c, 0, 0, 0);
+      }
+    }
+  };
+  int base = 0;
+  for (; base + U < nsteps; base += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      consume(u, base + u);
+      load_slot(u, base + u + U);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) consume(u, base + u);
+
+  // element i of lane l: row 16 mt + 4 (l / 16) + i, column 16 rb + l % 16
+  const int64_t n = rb * 16 + r;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float a[P];
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        a[p] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < NS; ++q) a[p] += acc[p][q][mt][i];
+      }
+      const int m = mt * 16 + 4 * g + i;
+      if (m >= M) continue;
+      if constexpr (MODE == KRQ_OUT_PARTIAL) {
+        reinterpret_cast<float*>(out)[((int64_t)sidx * M + m) * NO + n] = a[0];
+      } else if constexpr (MODE == KRQ_OUT_BF16) {
+        reinterpret_cast<uint16_t*>(out)[(int64_t)m * NO + n] = f32_to_bf16(a[0]);
+      } else {
+        const float gg = round_bf16(a[0]), uu = round_bf16(a[P - 1]);
+        const float sl = round_bf16(gg / (1.0f + expf(-gg)));
+        reinterpret_cast<uint16_t*>(out)[(int64_t)m * NO + n] = f32_to_bf16(sl * uu);
+      }
+    }
+}
+
 // The SwiGLU with its last column blocks split in half, as k_gemv_fp8_swiglu_mixed: workgroups
 // below nfull are two-matrix blocks, workgroup nfull + j is half-pair block 2 nfull + j (the same
 // steps per wave, so the same output bits).
@@ -445,6 +585,48 @@ bool launch_swiglu_mixed(int layout, int M, int64_t NO, int nw, size_t smem, hip
   return true;
 }
 
+// k_gemv_bf16_wide where it applies (false otherwise): launches of more than four rows whose replaced
+// plan has two waves, whole groups of four row blocks on at least half the compute units, the split's
+// activation rows within LDS. Four Qwen3-4B layers in one graph, us, 16-column blocks / wide, row-major
+// weights: M = 3 194.1 / 195.5 and M = 4 199.1 / 197.6 (left narrow), M = 6 202 / 190, M = 16 246 / 221, M = 32 336 / 256; packed: M = 16 205 / 189,
+// M = 32 291 / 229. Four slots: two measured 254 at M = 16 row-major, six 228, eight 234. The two-matrix
+// SwiGLU block (152 workgroups for gate_up) is wide above 16 rows only: at M = 16 23.8 us against
+// 25.2 wide, at M = 32 34.0 against 21.
+bool launch_wide(int layout, int M, int mode, int pb, int nw, int64_t NO, int split, hipStream_t s, const uint8_t* x,
+                 const uint8_t* w, int64_t K, int kts, void* out) {
+  const int64_t groups = NO / 16 / kWideRb;
+  const int kib = (kts + 1) / 2 * ((M + 7) / 8);  // LDS for the split's activation rows
+  if (M <= 4 || pb != 1 || nw != 2 || (NO / 16) % kWideRb != 0 || groups * split < 128 || kib > 160)
+    return false;
+  if (M * 2 * K > 0x7fffffff) return false;  // (32-bit activation offsets)
+  const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(split)), block(kWideRb * 64);
+#define KRQ_WIDE(MODE_, LAYOUT_, MT_, TL_) \
+  hipLaunchKernelGGL((k_gemv_bf16_wide<MODE_, LAYOUT_, MT_, 4, 2, TL_>), grid, block, 0, s, x, w, M, NO, K, kts, out)
+#define KRQ_WIDE_TL(MODE_, LAYOUT_, MT_)                     \
+  if (kib <= 40) { KRQ_WIDE(MODE_, LAYOUT_, MT_, 40); }      \
+  else if (kib <= 80) { KRQ_WIDE(MODE_, LAYOUT_, MT_, 80); } \
+  else { KRQ_WIDE(MODE_, LAYOUT_, MT_, 160); }
+#define KRQ_WIDE_M(MODE_, LAYOUT_) \
+  if (M <= 16) { KRQ_WIDE_TL(MODE_, LAYOUT_, 1) } else { KRQ_WIDE_TL(MODE_, LAYOUT_, 2) }
+#define KRQ_WIDE_L(MODE_)                                                    \
+  if (layout == KRQ_W_TILED) { KRQ_WIDE_M(MODE_, KRQ_W_TILED) } else { KRQ_WIDE_M(MODE_, KRQ_W_ROWMAJOR) }
+  if (mode == KRQ_OUT_PARTIAL) {
+    KRQ_WIDE_L(KRQ_OUT_PARTIAL)
+  } else if (mode == KRQ_OUT_BF16) {
+    KRQ_WIDE_L(KRQ_OUT_BF16)
+  } else if (mode == KRQ_OUT_SWIGLU && M > 16) {
+    if (layout == KRQ_W_TILED) { KRQ_WIDE_TL(KRQ_OUT_SWIGLU, KRQ_W_TILED, 2) }
+    else { KRQ_WIDE_TL(KRQ_OUT_SWIGLU, KRQ_W_ROWMAJOR, 2) }
+  } else {
+    return false;
+  }
+#undef KRQ_WIDE_L
+#undef KRQ_WIDE_M
+#undef KRQ_WIDE_TL
+#undef KRQ_WIDE
+  return true;
+}
+
 }  // namespace
 
 int krq::gemv_bf16_run(const void* x, const void* w, int w_layout, int64_t M, int64_t N, int64_t K,
@@ -480,6 +662,7 @@ int krq::gemv_bf16_run(const void* x, const void* w, int w_layout, int64_t M, in
   const uint8_t* wb = (const uint8_t*)w;
   const int m = static_cast<int>(M);
   hipStream_t s = (hipStream_t)stream;
+  if (launch_wide(w_layout, m, mode, pb, nw, NO, split, s, xb, wb, K, kts, out)) return krq_check_launch("gemv_bf16");
   if (mode == KRQ_OUT_BF16) launch_layout<KRQ_OUT_BF16>(w_layout, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
   else if (mode == KRQ_OUT_PARTIAL) launch_layout<KRQ_OUT_PARTIAL>(w_layout, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
   else if (mode == KRQ_OUT_SWIGLU && launch_swiglu_mixed(w_layout, m, NO, nw, smem, s, xb, wb, K, kts, out))

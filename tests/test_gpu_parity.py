@@ -867,6 +867,34 @@ def test_bf16_line_loads_equal_tiles(dev, M, N, K, split, swiglu):
     assert rel_err(y.sum(0) if split > 1 else y, ref) <= TOL
 
 
+# The wide BF16 blocks (whole groups of four row blocks) against the 16-column launch the same weights
+# with sixteen more output columns take: the shared columns bit for bit. Odd tile counts per split; rows
+# at the edges of the eight-row groups; LDS of each size up to 156 KiB; the SwiGLU above 16 rows.
+@pytest.mark.parametrize("M", [4, 5, 8, 9, 16, 17, 24, 25, 32])
+@pytest.mark.parametrize("N,K,split", [(2240, 4992, 4), (2240, 3968, 4), (2240, 9856, 4), (8192, 1248, 1),
+                                       (8192, 320, 0)])
+def test_bf16_wide_equals_narrow(dev, M, N, K, split):
+    from kernels import gemv as G
+    x, w = act(M, K, 80 + M).to(dev), weight(2 * N if split == 0 else N, K, 81).to(dev)
+    more = weight(16, K, 82).to(dev)
+    if split == 0:
+        wide = torch.cat([w[:N], more, w[N:], more])
+        pick, run = (lambda y: y[:, :N]), (lambda v: G.gemv_swiglu(x, v))
+    else:
+        wide = torch.cat([w, more])
+        pick, run = (lambda y: y[..., :N]), (lambda v: G.gemv(x, v, split))
+    y = run(w)
+    assert torch.equal(y, pick(run(wide)))
+    G.pack(w)
+    assert torch.equal(run(w), y)
+    ref = x.double() @ w.double().t()
+    if split == 0:
+        g, u = ref[:, :N].to(torch.bfloat16).double(), ref[:, N:].to(torch.bfloat16).double()
+        ref = torch.nn.functional.silu(g).to(torch.bfloat16).double() * u
+    got = y.double().sum(0) if split > 1 else y.double()
+    assert rel_err(got.cpu(), ref.cpu()) <= TOL
+
+
 @pytest.mark.parametrize("M", [1, 16])
 def test_lmhead_bf16_tiled(dev, M):
     from kernels import gemv as G
