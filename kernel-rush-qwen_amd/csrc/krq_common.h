@@ -170,7 +170,7 @@ KRQ_DEV float wave_sum(float v) {
 template <int NT>
 KRQ_DEV uint32_t block_max_u32(uint32_t v) {
   __shared__ uint32_t red[NT / kWave];
-  v = wave_max_u32(v);
+  v = wave_max_u32_dpp(v);
   const int w = threadIdx.x / kWave;
   if ((threadIdx.x & (kWave - 1)) == 0) red[w] = v;
   __syncthreads();
