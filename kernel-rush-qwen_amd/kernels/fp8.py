@@ -349,11 +349,13 @@ TILED_MIN_ROWS_SPLIT = {"given": 3, "token": 11}
 def _tiled_rows(x, a, xs, algo, least=TILED_MIN_ROWS):
     """bf16 rows at `least` <= M <= 32 go through quant_rows_tiled (scaled per token) or
     cast_tiled (a given scale) and the GEMV on tiled activations (the operands of quant_rows / _cast
-    + the row-major e4m3 GEMV, with contiguous loads); fewer rows, and rows longer than the tiled
-    kernels take, use the row-major kernels."""
+    + the row-major e4m3 GEMV, with contiguous loads); fewer rows, rows longer than the tiled
+    kernels take, and below TILED_MIN_ROWS rows that do not start on 16 bytes (the row-major
+    quantizers take any address) use the row-major kernels."""
     M, K = x.shape
     return (xs is None and x.dtype == torch.bfloat16 and least <= M <= DECODE_MAX_ROWS
-            and K % 64 == 0 and K <= TILED_ROWS_MAX_K and algo != L.ALGO_VALU)
+            and K % 64 == 0 and K <= TILED_ROWS_MAX_K and algo != L.ALGO_VALU
+            and (M >= TILED_MIN_ROWS or x.data_ptr() % 16 == 0))
 
 
 def _tiled_operand(x, a):

@@ -42,7 +42,8 @@ def _fp8_operands(h, w, a, h_layout):
     if ws.numel() == 1:          # linear_fp8's own ActScale over the whole of h
         a = _fp8.ActScale(h)
         return _fp8._cast(_fp8._rows(h), a), a.scale.reshape(1), 0, L.LM_FP8
-    tiled = h_layout == "tiled" or (h_layout == "auto" and M >= TILED_MIN_ROWS)
+    tiled = h_layout == "tiled" or (h_layout == "auto" and M >= TILED_MIN_ROWS
+                                    and (M >= _fp8.TILED_MIN_ROWS or h.data_ptr() % 16 == 0))
     if K % 64 == 0 and K <= _fp8.TILED_ROWS_MAX_K and tiled:   # tiled e4m3 rows
         h8, hs = _fp8.quant_rows_tiled(h)
         return h8, hs.reshape(-1), 1, L.LM_FP8_TILED_H
@@ -55,7 +56,8 @@ def lm_head_argmax(h, w, return_logits=False, h_layout="auto", a=None):
     fp8.quantize (per channel) or fp8.quantize_weight (per tensor). Returns int64 [M] token ids,
     or (ids, bf16 logits [M, V]) with return_logits=True. h_layout ("auto", "tiled" or
     "rowmajor"): how a per-channel FP8 head's per-token rows are laid out at M > 1 (the same
-    operands either way); "auto" takes tiled rows from TILED_MIN_ROWS. a: an ActScale / SharedScale for the FP8 head's activations (as
+    operands either way); "auto" takes tiled rows from TILED_MIN_ROWS (below fp8.TILED_MIN_ROWS: of
+    rows that start on 16 bytes). a: an ActScale / SharedScale for the FP8 head's activations (as
     linear_fp8 takes), instead of the scaling described in the module docstring."""
     L.require_device(h)
     M, K = h.shape

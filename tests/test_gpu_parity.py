@@ -932,3 +932,22 @@ def test_rows_longer_than_tiled_kernels_fall_back(dev, K):
     assert rel_err(lg.float().cpu().numpy(), yref) <= TOL
     ref_ids = O.argmax_lowest(O.bf16_to_f32(u16(lg)).reshape(M, N))  # the fold over its own logits
     assert np.array_equal(idx.cpu().numpy(), ref_ids)
+
+
+# Rows that do not start on 16 bytes, at the row counts that take tiled rows when they do: the row-major
+# quantizers, the same bits; from TILED_MIN_ROWS on they are refused.
+@pytest.mark.parametrize("M", [3, 5, 11, 12, 13])
+def test_unaligned_rows(dev, M):
+    K = 512
+    x = act(M, K, 90 + M).to(dev)
+    off = torch.empty(M * K + 1, dtype=torch.bfloat16, device=dev)[1:].view(M, K)
+    off.copy_(x)
+    q = fp8.quantize(weight(256, K, 91).to(dev))
+    a = fp8.ActScale(x, 2.0)
+    for run in (lambda v: fp8.gemv_fp8(v, q, 2), lambda v: fp8.gemv_fp8(v, q, 2, a=a),
+                lambda v: lmhead.lm_head_argmax(v, q, return_logits=True)[1]):
+        if M >= fp8.TILED_MIN_ROWS:
+            with pytest.raises(ValueError):
+                run(off)
+        else:
+            assert torch.equal(run(off), run(x))
