@@ -487,8 +487,7 @@ def linear_fp8(x, q, a=None, amax_out=None):
     128, K >= 256); the rest keep the reference's library GEMM, torch._scaled_mm (hipBLASLt on
     ROCm)."""
     w8, ws = q[0], q[1]
-    if (x.dim() == 2 and _cast is _cast_hip and _ring_gemm_fits(w8)
-            and x.shape[0] >= (PREFILL_MIN_ROWS if ws.numel() == 1 else PER_CHANNEL_MIN_ROWS)):
+    if x.dim() == 2 and x.shape[0] > DECODE_MAX_ROWS and _cast is _cast_hip and x.shape[0] >= _gemm_min_rows(w8, ws):
         return _linear_gemm(x, q, a, amax_out)
     x8 = None
     if a is None:
@@ -506,7 +505,7 @@ def linear_fp8(x, q, a=None, amax_out=None):
         x8 = _cast(x, a)
     if x.shape[0] <= DECODE_MAX_ROWS:
         return gemv_fp8_launch(x8, _one(a.scale), q, 1, L.OUT_BF16)
-    if x.shape[0] >= (PREFILL_MIN_ROWS if ws.numel() == 1 else PER_CHANNEL_MIN_ROWS) and _ring_gemm_fits(w8):
+    if x.shape[0] >= _gemm_min_rows(w8, ws):
         return gemm_fp8(x8, q, xs=_one(a.scale))
     return torch._scaled_mm(x8, w8.t(), scale_a=a.scale, scale_b=ws, out_dtype=torch.bfloat16)
 
@@ -517,6 +516,8 @@ def _linear_gemm(x, q, a, amax_out):
     host work (the launches take 3 us each): 37 us with an allocation per piece and the launches
     through ActScale and gemm_fp8, 20 us this way."""
     w8, ws = q[0], q[1]
+    if a is not None and a.scale.dtype != torch.float32:
+        raise ValueError("the activations' scale must be fp32")
     N, K = w8.shape
     x2 = _rows(x)
     M = x2.shape[0]
@@ -546,6 +547,16 @@ def _linear_gemm(x, q, a, amax_out):
     L.call("krq_gemm_fp8_ws", p + at8, L.X_FP8, scale, None, 0, L.ptr(w8), L.ptr(ws), 1 if ws.numel() > 1 else 0,
            M, N, K, p + at_split if split_bytes else None, split_bytes, L.ptr(out), st)
     return out
+
+
+def _gemm_min_rows(w8, ws):
+    """The rows from which linear_fp8 runs this library's GEMM on a weight. Below
+    PER_CHANNEL_MIN_ROWS what the library's product refuses (per-channel scales, scales that are
+    not fp32) or alone takes (a weight that does not start on 16 bytes) stays with it."""
+    if not _ring_gemm_fits(w8):
+        return float("inf")
+    own = ws.numel() == 1 and ws.dtype == torch.float32 and w8.data_ptr() % 16 == 0
+    return PREFILL_MIN_ROWS if own else PER_CHANNEL_MIN_ROWS
 
 
 def _ring_gemm_fits(w8):

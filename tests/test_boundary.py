@@ -215,3 +215,17 @@ def test_fused_and_gemm_wrappers_refuse_cpu_tensors():
         FG.gemv_fused(x, q, 1, ep=(x, x, x, x))
     with pytest.raises(RuntimeError, match="ROCm device"):
         fp8.gemm_fp8(torch.zeros(64, 256, dtype=torch.float8_e4m3fn), q, xs=torch.ones(1))
+
+
+def test_linear_gemm_rows():
+    """linear_fp8's line to this library's GEMM: one fp32 scale and an aligned weight from the first
+    row past the decode sizes, other weights of its shapes from PER_CHANNEL_MIN_ROWS, the rest never."""
+    w8 = torch.zeros(256 * 512 + 8, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    own, off = w8[:256 * 512].view(256, 512), w8[8:].view(256, 512)
+    assert own.data_ptr() % 16 == 0
+    one = torch.ones(())
+    assert fp8._gemm_min_rows(own, one) == fp8._gemm_min_rows(own, one.reshape(1)) == fp8.PREFILL_MIN_ROWS
+    for w, ws in ((off, one), (own, one.double()), (own, torch.ones(256))):
+        assert fp8._gemm_min_rows(w, ws) == fp8.PER_CHANNEL_MIN_ROWS
+    for w in (own[:, :128].contiguous(), own[:, :256], own[:200], own.view(torch.uint8)):
+        assert fp8._gemm_min_rows(w, one) == float("inf")

@@ -951,3 +951,10 @@ def test_unaligned_rows(dev, M):
                 run(off)
         else:
             assert torch.equal(run(off), run(x))
+
+
+def test_linear_fp8_scale_type(dev):
+    x, q = act(40, 512, 95).to(dev), fp8.quantize_weight(weight(256, 512, 96).to(dev))
+    a = fp8.ActScale(x)
+    with pytest.raises((RuntimeError, ValueError)):
+        fp8.linear_fp8(x, q, fp8.SharedScale(a.inv, a.scale.double()))
