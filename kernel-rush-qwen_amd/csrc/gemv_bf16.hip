@@ -244,6 +244,8 @@ __global__ __launch_bounds__(512) void k_gemv_bf16(const uint8_t* __restrict__ x
 // streams only its weights through a ring of U step slots. Steps, products and sums are those of the
 // NS-wave launch it replaces: step j goes to accumulator set j % NS, the sets are added from zero in
 // wave order, so the results are the same bit for bit.
+// (The two sets on two waves, eight waves a workgroup with the sets added through LDS, measured
+// slower: four layers row-major, M = 16 221.5 -> 226 us, M = 32 247.5 -> 254.8; packed M = 32 229 -> 242.)
 // LDS: step j of row group h (rows 8 h .. 8 h + 7 of the HV in use) is 1 KiB at (j HV + h) KiB, entry
 // 8 (c ^ (h % 2)) + row the row's 16-byte chunk c: a wave's operand read (rows 0-7 of one group, 8-15 of
 // the next, one chunk) then covers 256 consecutive bytes modulo the banks.
@@ -280,7 +282,7 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* 
              lx + 1024u * static_cast<uint32_t>(i));
   }
   uint4 wl[P][U], wh[P][U];
-  auto load_slot = [&](int u, int cc) {  // (a slot past the last step reloads it, masked where consumed)
+  auto load_slot = [&](int u, int cc) {  // (a slot past the last step reloads it and is not consumed)
     const int j = min(cc, nsteps - 1);
     const int64_t t0 = tbase + 2 * j, t1 = (2 * j + 1 < kts) ? t0 + 1 : t0;
 #pragma unroll
@@ -313,9 +315,8 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* 
     for (int q = 0; q < NS; ++q)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[p][q][mt] = v4f{0.f, 0.f, 0.f, 0.f};
-  auto consume = [&](int u, int cc) {
-    const int j = min(cc, nsteps - 1);
-    const bool ok = cc < nsteps, hi = ok && (2 * j + 1 < kts);
+  auto consume = [&](int u, int j) {
+    const bool hi = 2 * j + 1 < kts;
     uint4 al[MT], ah[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {  // (rows past the groups in use read the last group)
@@ -328,7 +329,6 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* 
     for (int p = 0; p < P; ++p) {
       uint4 bl = wl[p][u], bh = wh[p][u];
       if constexpr (RM) lines_to_tiles(wl[p][u], wh[p][u], &bl, &bh);
-      bl = sel4(ok, bl);
       bh = sel4(hi, bh);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
@@ -348,7 +348,8 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* 
     }
   }
 #pragma unroll
-  for (int u = 0; u < U; ++u) consume(u, base + u);
+  for (int u = 0; u < U; ++u)
+    if (base + u < nsteps) consume(u, base + u);  // (not zeroed weights: an infinite activation times them is NaN)
 
   // element i of lane l: row 16 mt + 4 (l / 16) + i, column 16 rb + l % 16
   const int64_t n = rb * 16 + r;

@@ -298,3 +298,21 @@ def test_fp8_lm_head_nan_row_argmax_first(dev):
     idx, logits = lmhead.lm_head_argmax(h.to(dev), q, return_logits=True)
     assert torch.isnan(logits.float()).all()
     assert idx.item() == 0 == torch.argmax(logits.float(), -1).item()
+
+
+# An infinite activation in the last step of K, at every remainder of the wide BF16 blocks' four-step
+# rounds: infinite outputs of the products' signs there, no other row touched. (Odd counts of steps: the
+# two-wave blocks that other grids run reload only the second wave's last step.)
+@pytest.mark.parametrize("steps", [7, 11, 16])
+@pytest.mark.parametrize("M", [5, 16, 32])
+def test_bf16_infinity_in_the_last_step(dev, M, steps):
+    from kernels.gemv import gemv
+    g = torch.Generator().manual_seed(97)
+    K = 64 * steps
+    w = (torch.randn(8192, K, generator=g) * 0.02).to(torch.bfloat16)
+    w[:, -1] = torch.where(w[:, -1] == 0, 0.01, w[:, -1].float()).to(torch.bfloat16)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    x[M - 1, -1] = float("inf")
+    y = gemv(x.to(dev), w.to(dev), 1).float().cpu()
+    assert torch.equal(y[M - 1], torch.full((8192,), float("inf")) * torch.sign(w[:, -1].float()))
+    assert torch.isfinite(y[:M - 1]).all()
