@@ -168,7 +168,7 @@ def _cast_hip(x, a):
     M, K = x2.shape
     L.require_device(a.inv)
     y = torch.empty(x.shape, device=x.device, dtype=torch.float8_e4m3fn)
-    L.call("krq_cast_fp8", L.ptr(x2), M, K, L.ptr(a.inv), 0, L.ptr(y), L.stream(x2))
+    L.call("krq_cast_fp8", L.ptr(x2), M, K, L.ptr(_one(a.inv)), 0, L.ptr(y), L.stream(x2))
     return y
 
 
@@ -228,12 +228,17 @@ def pick_cast(log):
 # ---------------------------------------------------------------------------------------------
 # skinny GEMM / GEMV
 # ---------------------------------------------------------------------------------------------
+def _check_weight_scale(ws, N):
+    """The kernels read a weight's scale as one fp32 value or one per output row."""
+    if ws.dtype != torch.float32 or ws.numel() not in (1, N) or not ws.is_contiguous():
+        raise ValueError(f"weight scale must be contiguous fp32 with 1 or {N} values, got {ws.dtype} {tuple(ws.shape)}")
+
+
 def _weight_operand(q):
     w8, ws = q[0], q[1]
     tiled = getattr(q, "tiled", None)
     L.require_device(w8, ws)
-    if ws.dtype != torch.float32:
-        raise ValueError("weight scale must be fp32")
+    _check_weight_scale(ws, w8.shape[0])
     if tiled is not None:
         return tiled, L.W_TILED, ws, w8.shape
     if w8.dtype != torch.float8_e4m3fn or w8.dim() != 2 or not w8.is_contiguous():
@@ -300,7 +305,9 @@ def gemv_fp8_bf16_launch(x, q, split=1, mode=L.OUT_BF16, a=None, algo=L.ALGO_AUT
 
 
 def _one(scale):
-    """A per-tensor scale as the launches take it: one value (0-d or [1])."""
+    """A per-tensor scale (or its inverse) as the launches take it: one fp32 value (0-d or [1])."""
+    if scale.dtype != torch.float32:
+        raise ValueError(f"activation scales must be fp32, got {scale.dtype}")
     return scale if scale.numel() == 1 else scale.reshape(1)
 
 
@@ -324,6 +331,8 @@ def _activation_fp8(x, a, xs):
     if x.dtype == torch.float8_e4m3fn:
         if xs is None:
             raise ValueError("float8 activations need their scale xs")
+        if xs.dtype != torch.float32 or xs.numel() not in (1, x.shape[0]):
+            raise ValueError("xs must be fp32 with 1 or M values")
         return x.contiguous(), xs.reshape(-1).contiguous()
     if a is not None:
         return _cast(x, a), _one(a.scale)
@@ -437,8 +446,8 @@ def swiglu_cast_fp8(x, q, out_a, a=None, xs=None):
     MP = 16 * ((M + 15) // 16)
     x8t = torch.empty((MP * (N // 2),), device=x.device, dtype=torch.uint8)
     L.call("krq_gemv_swiglu_fp8_cast", L.ptr(xin), kind, L.ptr(x_scale), L.ptr(x_inv), xpr, L.ptr(w), layout,
-           L.ptr(ws), 1 if ws.numel() > 1 else 0, M, N, K, L.ptr(out_a.inv.reshape(1)), L.ptr(x8t), L.stream(x))
-    return x8t, out_a.scale.reshape(1)
+           L.ptr(ws), 1 if ws.numel() > 1 else 0, M, N, K, L.ptr(_one(out_a.inv)), L.ptr(x8t), L.stream(x))
+    return x8t, _one(out_a.scale).reshape(1)
 
 
 def gemm_fp8(x, q, a=None, xs=None):
@@ -454,6 +463,7 @@ def gemm_fp8(x, q, a=None, xs=None):
     if w8.dtype != torch.float8_e4m3fn or w8.dim() != 2 or not w8.is_contiguous():
         raise ValueError("expected a contiguous float8_e4m3fn [N, K] weight")
     N, K = w8.shape
+    _check_weight_scale(ws, N)
     if x.dim() != 2 or x.shape[1] != K:
         raise ValueError(f"x {tuple(x.shape)} does not match w8 {tuple(w8.shape)}")
     M = x.shape[0]
@@ -516,9 +526,11 @@ def _linear_gemm(x, q, a, amax_out):
     host work (the launches take 3 us each): 37 us with an allocation per piece and the launches
     through ActScale and gemm_fp8, 20 us this way."""
     w8, ws = q[0], q[1]
-    if a is not None and a.scale.dtype != torch.float32:
-        raise ValueError("the activations' scale must be fp32")
     N, K = w8.shape
+    _check_weight_scale(ws, N)
+    if a is not None:
+        inv, given = _one(a.inv), _one(a.scale)
+        L.require_device(inv, given)
     x2 = _rows(x)
     M = x2.shape[0]
     L.require_device(w8, ws)
@@ -541,9 +553,8 @@ def _linear_gemm(x, q, a, amax_out):
         if amax_out is not None:
             amax_out.copy_(torch.maximum(amax_out, work[:4].view(torch.float32)))
     else:
-        L.require_device(a.inv, a.scale)
-        scale = L.ptr(_one(a.scale))
-        L.call("krq_cast_fp8", L.ptr(x2), M, K, L.ptr(a.inv), 0, p + at8, st)
+        scale = L.ptr(given)
+        L.call("krq_cast_fp8", L.ptr(x2), M, K, L.ptr(inv), 0, p + at8, st)
     L.call("krq_gemm_fp8_ws", p + at8, L.X_FP8, scale, None, 0, L.ptr(w8), L.ptr(ws), 1 if ws.numel() > 1 else 0,
            M, N, K, p + at_split if split_bytes else None, split_bytes, L.ptr(out), st)
     return out

@@ -152,14 +152,14 @@ def _launch_fp8(x, q, split, mode, norm, ep, eps, a, out):
                 return _fp8.gemv_fp8_tiled_launch(x8, xs, q, M, split, mode, out)
             if tiled:
                 x8t = _fp8.cast_tiled(_rmsnorm(x, ln, ss, eps), a)
-                return _fp8.gemv_fp8_tiled_launch(x8t, a.scale.reshape(1), q, M, split, mode, out)
+                return _fp8.gemv_fp8_tiled_launch(x8t, _fp8._one(a.scale), q, M, split, mode, out)
             if a is None:
                 x8 = torch.empty((M, K), device=x.device, dtype=torch.float8_e4m3fn)
                 xs = torch.empty((M,), device=x.device, dtype=torch.float32)
                 L.call("krq_rmsnorm_quant_rows", L.ptr(x), L.ptr(ss), L.ptr(ln), float(eps), M, K, L.ptr(x8),
                        L.ptr(xs), L.stream(x))
             else:
-                x8, xs = _fp8._cast(_rmsnorm(x, ln, ss, eps), a), a.scale.reshape(1)
+                x8, xs = _fp8._cast(_rmsnorm(x, ln, ss, eps), a), _fp8._one(a.scale)
             return _fp8.gemv_fp8_launch(x8, xs, q, split, mode, L.ALGO_MFMA, out)
         if tiled:
             x8, xs = _fp8._tiled_operand(x, a)
@@ -168,7 +168,7 @@ def _launch_fp8(x, q, split, mode, norm, ep, eps, a, out):
             x8, xs = _fp8._activation_fp8(x, a, None)
             kind, xin, x_scale, x_inv = L.X_FP8, x8, xs, None
     elif a is not None:
-        xin, x_scale, x_inv = x, a.scale.reshape(1), a.inv.reshape(1)
+        xin, x_scale, x_inv = x, _fp8._one(a.scale), _fp8._one(a.inv)
     else:
         xin, x_scale, x_inv = x, None, None
     xpr = 1 if (x_scale is not None and x_scale.numel() == M and M > 1) else 0

@@ -32,11 +32,10 @@ def _fp8_operands(h, w, a, h_layout):
     M, K = h.shape
     V = w[0].shape[0]
     ws = w[1]
-    if ws.numel() not in (1, V):
-        raise ValueError("the FP8 lm head needs per-channel or per-tensor weight scales")
+    _fp8._check_weight_scale(ws, V)
     if a is not None:            # a given scale: linear_fp8(h, q, a)
         h8 = _fp8._cast(_fp8._rows(h), a)
-        return h8, a.scale.reshape(1), 0, L.LM_FP8
+        return h8, _fp8._one(a.scale), 0, L.LM_FP8
     if M == 1:                   # per token == per tensor: scaled inside the GEMV
         return _fp8._rows(h), None, 0, L.LM_FP8
     if ws.numel() == 1:          # linear_fp8's own ActScale over the whole of h

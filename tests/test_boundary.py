@@ -229,3 +229,24 @@ def test_linear_gemm_rows():
         assert fp8._gemm_min_rows(w, ws) == fp8.PER_CHANNEL_MIN_ROWS
     for w in (own[:, :128].contiguous(), own[:, :256], own[:200], own.view(torch.uint8)):
         assert fp8._gemm_min_rows(w, one) == float("inf")
+
+
+def test_scales_are_fp32_of_the_right_count():
+    """The kernels read scales through float pointers: another type, another number of values or
+    strided ones are refused before any launch (and before the device is looked at)."""
+    N, K = 256, 512
+    w8 = torch.zeros(N, K, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    x = torch.zeros(128, K, dtype=torch.bfloat16)
+    good = torch.ones(())
+    for ws in (good.double(), torch.ones(N).bfloat16(), torch.ones(7), torch.ones(2 * N)[::2], good.expand(N)):
+        with pytest.raises(ValueError, match="weight scale"):
+            fp8._check_weight_scale(ws, N)
+        with pytest.raises(ValueError, match="weight scale"):
+            fp8.linear_fp8(x, (w8, ws))
+    for ws in (good, good.reshape(1), torch.ones(N), torch.ones(N, 1)):
+        fp8._check_weight_scale(ws, N)
+    for a in (fp8.SharedScale(good, good.double()), fp8.SharedScale(good.bfloat16(), good)):
+        with pytest.raises(ValueError, match="fp32"):
+            fp8.linear_fp8(x, (w8, good), a)
+    with pytest.raises(ValueError, match="fp32"):
+        fp8._activation_fp8(x.to(torch.float8_e4m3fn), None, good.double())

@@ -230,3 +230,23 @@ def test_gemm_rejects_bad_shapes(dev):
     x8, xs = F.quant_rows(bf((64, 256), 8).to(dev))
     with pytest.raises(ValueError):
         F.gemm_fp8(x8, q, xs=xs)
+
+
+@pytest.mark.parametrize("M", [1, 5, 16, 33, 128])
+def test_scales_refused(dev, M):
+    """Scales of another type or count than the kernels read, from every row count's route."""
+    q = F.quantize_weight(bf((256, 512), 56, 0.02).to(dev))
+    x = bf((M, 512), 57).to(dev)
+    a = F.ActScale(x)
+    for ws in (q[1].double(), q[1].repeat(3)):
+        bad = F.FP8Weight(q[0], ws, q.tiled)
+        with pytest.raises((RuntimeError, ValueError)):
+            F.linear_fp8(x, bad)
+        with pytest.raises(ValueError):
+            F.gemm_fp8(x, bad, a)
+        if M <= 32:
+            with pytest.raises(ValueError):
+                F.gemv_fp8(x, bad, 2)
+    for s in (F.SharedScale(a.inv.double(), a.scale), F.SharedScale(a.inv, a.scale.double())):
+        with pytest.raises((RuntimeError, ValueError)):
+            F.linear_fp8(x, q, s)
