@@ -360,10 +360,12 @@ def _tiled_rows(x, a, xs, algo, least=TILED_MIN_ROWS):
     cast_tiled (a given scale) and the GEMV on tiled activations (the operands of quant_rows / _cast
     + the row-major e4m3 GEMV, with contiguous loads); fewer rows, rows longer than the tiled
     kernels take, and below TILED_MIN_ROWS rows that do not start on 16 bytes (the row-major
-    quantizers take any address) use the row-major kernels."""
+    quantizers take any address) use the row-major kernels, as do given-scale rows where pick_cast
+    has put torch's cast in the place of the HIP one."""
     M, K = x.shape
     return (xs is None and x.dtype == torch.bfloat16 and least <= M <= DECODE_MAX_ROWS
             and K % 64 == 0 and K <= TILED_ROWS_MAX_K and algo != L.ALGO_VALU
+            and (a is None or _cast is _cast_hip)
             and (M >= TILED_MIN_ROWS or x.data_ptr() % 16 == 0))
 
 

@@ -142,7 +142,8 @@ def _launch_fp8(x, q, split, mode, norm, ep, eps, a, out):
     if not fits(M, N, K, split, mode, kind, 1 if norm is not None else 0):
         # stage outside: normalize (and quantize) the rows first, then e4m3 activations, row-major
         # or (from fp8.TILED_MIN_ROWS rows) in the tiled activation layout, as fp8's GEMVs choose
-        tiled = K % 64 == 0 and K <= _fp8.TILED_ROWS_MAX_K and M >= _fp8.TILED_MIN_ROWS
+        tiled = K % 64 == 0 and K <= _fp8.TILED_ROWS_MAX_K and M >= _fp8.TILED_MIN_ROWS and (
+            a is None or _fp8._cast is _fp8._cast_hip)
         if norm is not None:
             if tiled and a is None:
                 x8 = torch.empty(((M + 15) // 16 * 16 * K,), device=x.device, dtype=torch.uint8)

@@ -250,3 +250,13 @@ def test_scales_are_fp32_of_the_right_count():
             fp8.linear_fp8(x, (w8, good), a)
     with pytest.raises(ValueError, match="fp32"):
         fp8._activation_fp8(x.to(torch.float8_e4m3fn), None, good.double())
+
+
+def test_given_scale_rows_keep_the_picked_cast(monkeypatch):
+    """Rows with a given scale take the tiled cast kernel only while pick_cast keeps the HIP cast."""
+    a = fp8.SharedScale(torch.ones(1), torch.ones(()))
+    x = {M: torch.zeros(M, 256, dtype=torch.bfloat16) for M in (3, 12, 13, 32)}
+    assert all(fp8._tiled_rows(v, a, None, L.ALGO_AUTO, 3) for v in x.values())
+    monkeypatch.setattr(fp8, "_cast", fp8._cast_torch)
+    assert not any(fp8._tiled_rows(v, a, None, L.ALGO_AUTO, 3) for v in x.values())
+    assert all(fp8._tiled_rows(v, None, None, L.ALGO_AUTO, 3) for v in x.values())

@@ -958,3 +958,23 @@ def test_linear_fp8_scale_type(dev):
     a = fp8.ActScale(x)
     with pytest.raises((RuntimeError, ValueError)):
         fp8.linear_fp8(x, q, fp8.SharedScale(a.inv, a.scale.double()))
+
+
+# pick_cast's fallback (torch's cast) serves every GEMV that casts its rows first, whatever their number
+@pytest.mark.parametrize("M", [2, 5, 12, 16, 32])
+def test_picked_cast_is_used(dev, M, monkeypatch):
+    K, N = 512, 256
+    x, q = act(M, K, 97 + M).to(dev), fp8.quantize(weight(N, K, 98).to(dev))
+    a = fp8.ActScale(x, 2.0)
+    calls = (lambda: fp8.gemv_fp8(x, q, 2, a=a), lambda: fp8.gemv_fp8(x, q, 1, a=a),
+             lambda: fp8.gemv_swiglu_fp8(x, q, a=a), lambda: fp8.linear_fp8(x, q, a))
+    want = [f() for f in calls]
+    seen = []
+
+    def picked(v, s):
+        seen.append(v.shape)
+        return fp8._cast_torch(v, s)
+
+    monkeypatch.setattr(fp8, "_cast", picked)
+    for i, f in enumerate(calls):
+        assert torch.equal(f(), want[i]) and len(seen) == i + 1, i
