@@ -148,6 +148,9 @@ int krq_gemv_fp8(const void* x, int x_kind, const float* x_scale, const float* x
                  const void* w8, int w_layout, const float* w_scale, int w_per_row,
                  int64_t M, int64_t N, int64_t K, int split, int mode, int algo,
                  void* out, void* stream);
+/* 1 where krq_gemv_fp8 on KRQ_X_FP8_TILED rows (KRQ_OUT_BF16 or KRQ_OUT_PARTIAL, 2 <= M <= 16) runs
+ * the launch whose workgroups share the rows in LDS, else 0: with it the tiled rows pay from fewer rows. */
+int64_t krq_gemv_fp8_shares_rows(int64_t M, int64_t N, int64_t K, int split, int w_layout);
 
 /*
  * The FP8 SwiGLU GEMV with the next projection's input cast in its epilogue: the engine's
@@ -211,6 +214,9 @@ int krq_lmhead_argmax(const void* h, const float* h_scale, int h_per_row, const 
                       int w_layout, const float* w_scale, int w_per_row, int64_t M, int64_t V, int64_t K,
                       void* logits, void* ws, int64_t ws_bytes, int64_t* idx_out, void* stream);
 int64_t krq_lmhead_ws_bytes(int64_t M, int64_t V);
+/* 1 where KRQ_LM_FP8_TILED_H runs the persistent launch that keeps h's tiles in LDS, on a grid that
+ * fills the chip (2 <= M <= 16), else 0: with it the tiled rows pay from fewer rows. */
+int64_t krq_lmhead_shares_rows(int64_t M, int64_t V, int64_t K, int w_layout);
 
 /*
  * krq_lmhead_argmax without the workspace argument: the call allocates nothing. No counterpart in

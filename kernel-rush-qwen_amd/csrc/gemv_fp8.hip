@@ -378,19 +378,24 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_wide32(const uint8_t* __r
   KRQ_STAMP(3, threadIdx.x == 0);
 }
 
+// The shapes the wide-block launch takes: one row block per block in the plan (pb 1) and ns <= 4 waves
+// per row block, row blocks a multiple of kWideRb, the split's tiles within LDS.
+bool wide32_shape(int64_t M, int pb, int ns, int64_t NO, int kts) {
+  return pb == 1 && ns >= 1 && ns <= 4 && (NO / 16) % kWideRb == 0 && (M > 16 ? 2 : 1) * kts <= 96;
+}
+
 // The wide-block launch when it applies (1 < M <= 32, tiled e4m3 rows and tiled weights, the
-// plain output modes, one row block per block in the plan (pb 1) and ns <= 4 waves per row block,
-// row blocks a multiple of kWideRb, the split's tiles within LDS); false otherwise.
+// plain output modes, wide32_shape); false otherwise.
 bool launch_wide32(int M, int mode, int x_kind, int w_layout, int algo, const void* aux, int pb, int ns, int64_t NO,
                    int split, int kts, hipStream_t s, const uint8_t* xb, const float* x_scale, int x_per_row,
                    const uint8_t* wb, const float* w_scale, int w_per_row, int64_t K, void* out) {
   // (at M = 16, graph-timed: down 7.48 -> 7.03 us, QKV 4.87 -> 4.66, O 4.52 -> 4.20 with eight
   // slots for its eight steps; ten, two of them masked, measured 4.57)
-  if (M < 2 || M > 32 || x_kind != KRQ_X_FP8_TILED || w_layout != KRQ_W_TILED || algo != 1 || pb != 1) return false;
+  if (M < 2 || M > 32 || x_kind != KRQ_X_FP8_TILED || w_layout != KRQ_W_TILED || algo != 1) return false;
   // (the two-matrix SwiGLU block measured slower wide: gate_up 12.7 -> 15.1 us at 254 VGPRs)
   if (!(mode == KRQ_OUT_PARTIAL || mode == KRQ_OUT_BF16)) return false;
+  if (!wide32_shape(M, pb, ns, NO, kts)) return false;
   const int mt = M > 16 ? 2 : 1;  // activation row tiles
-  if ((NO / 16) % kWideRb != 0 || mt * kts > 96 || ns < 1 || ns > 4) return false;
   const dim3 grid(static_cast<unsigned>(NO / 16 / kWideRb), static_cast<unsigned>(split)), block(kWideRb * 64);
   const int m = M;
   // slots: a multiple of the sets, ten at most (two-matrix blocks take 254 VGPRs with ten); one
@@ -564,6 +569,13 @@ bool launch_wide1(int M, int mode, int x_kind, int w_layout, int algo, int pb, i
   return true;
 }
 
+// Paired row blocks for the multi-row matrix-core kernels. Measured: pairing halves the blocks,
+// which costs the Qwen3-4B projections (640-768 blocks) more than the saved activation reads
+// gain; the lm_head (9,496 blocks) gains 10-15%.
+int row_blocks(int64_t M, int mode, int algo, int64_t NO, int split) {
+  return mode != KRQ_OUT_SWIGLU && algo != 2 && M > 4 && (NO / 16) % 2 == 0 && (NO / 16) * split >= 4096 ? 2 : 1;
+}
+
 // Activation-wave chunks per lane holding `span` bf16 elements (0: too long for one wave).
 int aw_chunks(int64_t span) {
   return span <= 512 * kAwRow ? kAwRow : span <= 512 * kAwSmall ? kAwSmall : span <= 512 * kAwLarge ? kAwLarge : 0;
@@ -610,11 +622,7 @@ int krq::gemv_fp8_run(const void* x, int x_kind, const float* x_scale, const flo
   const uint8_t* wb = (const uint8_t*)w8;
   const int m = static_cast<int>(M);
   hipStream_t s = (hipStream_t)stream;
-  // Paired row blocks for the multi-row matrix-core kernels. Measured: pairing halves the blocks,
-  // which costs the Qwen3-4B projections (640-768 blocks) more than the saved activation reads
-  // gain; the lm_head (9,496 blocks) gains 10-15%.
-  const int pb = (mode != KRQ_OUT_SWIGLU && algo != 2 && M > 4 && (NO / 16) % 2 == 0 &&
-                  (NO / 16) * split >= 4096) ? 2 : 1;
+  const int pb = row_blocks(M, mode, algo, NO, split);
   const int P = mode == KRQ_OUT_SWIGLU ? 2 : pb;
   const int MT = (algo == 2 || M <= 16) ? 1 : 2;
   const int64_t blocks = NO / 16 / pb * split;
@@ -728,6 +736,16 @@ extern "C" int krq_gemv_fp8(const void* x, int x_kind, const float* x_scale, con
   KRQ_REQUIRE(mode >= KRQ_OUT_BF16 && mode <= KRQ_OUT_SWIGLU, "gemv_fp8: bad mode %d", mode);
   return gemv_fp8_run(x, x_kind, x_scale, x_inv, x_per_row, w8, w_layout, w_scale, w_per_row, M, N,
                       K, split, mode, algo, out, nullptr, stream);
+}
+
+extern "C" int64_t krq_gemv_fp8_shares_rows(int64_t M, int64_t N, int64_t K, int split, int w_layout) {
+  if (M < 2 || M > 16 || w_layout != KRQ_W_TILED || N <= 0 || N % 16 != 0 || K <= 0 || split < 1 || K % split != 0 ||
+      (K / split) % 64 != 0 || K / split / 64 > 0x7fffffff)
+    return 0;
+  const int kts = static_cast<int>(K / split / 64);
+  int u = 0, nw = 0;
+  rows_ring((kts + 1) / 2, 1, &u, &nw);  // (krq_gemv_fp8's plan at M <= 16)
+  return wide32_shape(M, row_blocks(M, KRQ_OUT_BF16, 1, N, split), nw, N, kts);
 }
 
 extern "C" int krq_gemv_swiglu_fp8_cast(const void* x, int x_kind, const float* x_scale, const float* x_inv,

@@ -287,24 +287,39 @@ int lmhead_check(const void* h, const float* h_scale, const void* w, int w_kind,
   return KRQ_OK;
 }
 
+// The persistent kernel's (k_lmhead_fp8_persist) grid and ring for tiled e4m3 h: tiled weights, one row
+// tile, h's tile row within LDS, steps a multiple of the ring; its candidates are [M][its waves].
+// blocks 0: the shape runs the one-launch-per-row-block kernel.
+struct PersistPlan {
+  int64_t blocks;
+  int ring;
+};
+PersistPlan persist_plan(int64_t M, int64_t V, int64_t K, int w_layout) {
+  const int64_t nrb = V / 16, nsteps = K / 128;
+  const int ring = nsteps % 10 == 0 ? 10 : nsteps % 8 == 0 ? 8 : 0;
+  // at most one wave per row block: ncand <= nrb candidates per token fit krq_lmhead_ws_bytes
+  const int64_t blocks = std::min<int64_t>(kPersistBlocks, nrb / kPersistWaves);
+  const int64_t ncand = blocks * kPersistWaves;
+  if (w_layout != KRQ_W_TILED || M > 16 || blocks <= 0 || K <= 0 || K % 128 != 0 || K > kPersistMaxK || ring == 0 ||
+      (nrb + ncand - 1) / ncand > kPersistMaxRows)
+    return {0, 0};
+  return {blocks, ring};
+}
+
+// h's tile row, then each wave's table of column scales
+size_t persist_smem(int64_t K) { return 16 * (size_t)K + sizeof(float) * kPersistWaves * kPersistMaxRows * 16; }
+
 // The two launches into the candidate buffer ws (krq_lmhead_ws_bytes(M, V) bytes, all of which the
 // GEMV writes before the fold reads them: nothing needs clearing between calls).
 int lmhead_launch(const void* h, const float* h_scale, int h_per_row, const void* w, int w_kind, int w_layout,
                   const float* w_scale, int w_per_row, int64_t M, int64_t V, int64_t K, void* logits, void* ws,
                   int64_t* idx_out, void* stream) {
   int rc;
-  // tiled e4m3 h and tiled weights, one row tile, h's tile row within LDS, steps a multiple of the
-  // ring: the persistent kernel (k_lmhead_fp8_persist), its candidates [M][its waves]
-  const int64_t nrb = V / 16, nsteps = K / 128;
-  const int ring = nsteps % 10 == 0 ? 10 : nsteps % 8 == 0 ? 8 : 0;
-  // at most one wave per row block: ncand <= nrb candidates per token fit krq_lmhead_ws_bytes
-  const int64_t blocks = std::min<int64_t>(kPersistBlocks, nrb / kPersistWaves);
-  const int64_t ncand = blocks * kPersistWaves;
-  if (w_kind == KRQ_LM_FP8_TILED_H && w_layout == KRQ_W_TILED && M <= 16 && blocks > 0 && K % 128 == 0 &&
-      K <= kPersistMaxK && ring > 0 && (nrb + ncand - 1) / ncand <= kPersistMaxRows && aligned16(h) &&
-      aligned16(w)) {
-    // h's tile row, then each wave's table of column scales
-    const size_t smem = 16 * (size_t)K + sizeof(float) * kPersistWaves * kPersistMaxRows * 16;
+  const PersistPlan pp = persist_plan(M, V, K, w_layout);
+  if (w_kind == KRQ_LM_FP8_TILED_H && pp.blocks > 0 && aligned16(h) && aligned16(w)) {
+    const int64_t blocks = pp.blocks, ncand = blocks * kPersistWaves;
+    const int ring = pp.ring;
+    const size_t smem = persist_smem(K);
     hipStream_t s = (hipStream_t)stream;
 #define KRQ_PERSIST(UV, SV)                                                                                     \
   hipLaunchKernelGGL((k_lmhead_fp8_persist<UV, SV>), dim3(static_cast<unsigned>(blocks)), dim3(kPersistWaves * 64), \
@@ -343,6 +358,16 @@ int lmhead_launch(const void* h, const float* h_scale, int h_per_row, const void
 }
 
 }  // namespace
+
+// Where the persistent kernel also fills the chip: at least three quarters of its full grid, and two
+// workgroups within a unit's LDS. Below that, tiled rows measured slower (M = 5 and 8, us row-major /
+// tiled): V = 16,448, K = 2,560 16.0 / 17.9 and 16.5 / 18.0 (V = 24,576, K = 2,048 17.7 / 17.8 and 18.6
+// / 17.9, V = 32,000, K = 4,096 30.1 / 30.4 and 32.3 / 30.5); K = 8,192, one workgroup per unit, V =
+// 128,256 177.5 / 181.3 and 180.1 / 182.2.
+extern "C" int64_t krq_lmhead_shares_rows(int64_t M, int64_t V, int64_t K, int w_layout) {
+  return M >= 2 && V > 0 && persist_plan(M, V, K, w_layout).blocks >= kPersistBlocks / 4 * 3 &&
+         2 * persist_smem(K) <= 160 * 1024;
+}
 
 extern "C" int krq_lmhead_argmax(const void* h, const float* h_scale, int h_per_row, const void* w,
                                  int w_kind, int w_layout, const float* w_scale, int w_per_row, int64_t M,

@@ -36,6 +36,7 @@ EXPORTS = {
     "krq_cast_fp8_tiled": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp]),
     "krq_gemv_fp8": (_i32, [_vp, _i32, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _i64, _i64,
                             _i32, _i32, _i32, _vp, _vp]),
+    "krq_gemv_fp8_shares_rows": (_i64, [_i64, _i64, _i64, _i32, _i32]),
     "krq_gemv_swiglu_fp8_cast": (_i32, [_vp, _i32, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _i64, _i64,
                                         _vp, _vp, _vp]),
     "krq_gemv_bf16": (_i32, [_vp, _vp, _i32, _i64, _i64, _i64, _i32, _i32, _vp, _vp]),
@@ -43,6 +44,7 @@ EXPORTS = {
     "krq_lmhead_argmax": (_i32, [_vp, _vp, _i32, _vp, _i32, _i32, _vp, _i32, _i64, _i64, _i64, _vp, _vp,
                                  _i64, _vp, _vp]),
     "krq_lmhead_ws_bytes": (_i64, [_i64, _i64]),
+    "krq_lmhead_shares_rows": (_i64, [_i64, _i64, _i64, _i32]),
     "krq_lmhead_argmax_noalloc": (_i32, [_vp, _vp, _i32, _vp, _i32, _i32, _vp, _i32, _i64, _i64, _i64, _vp,
                                          _vp, _vp]),
     "krq_mlp_fp8": (_i32, [_vp, _i32, _vp, _vp, _i32, _vp, _i32, _vp, _vp, _i32, _i64, _i64, _i64,

@@ -346,13 +346,29 @@ def _activation_fp8(x, a, xs):
 # 7.52 / 7.40; gate_up M = 4 12.64 / 13.47, M = 16 14.19 / 13.70; down M = 4 9.70 / 10.35, M = 16
 # 11.24 / 10.83; given scale M = 8 QKV 7.19 / 7.60, M = 16 8.25 / 7.68, M = 32 10.47 / 9.29.
 TILED_MIN_ROWS = 13
-# Split-K GEMVs take the tiled rows earlier: their workgroups share them in LDS (k_gemv_wide32), where
-# one K pass over a whole row measures slower on them below 13 rows (linear_fp8 over a layer's four
-# projections at M = 5 36.4 us row-major, 43.0 tiled). With a given scale from three rows, scaled per
-# token from ten (QKV, O, gate_up and down of eight layers in one graph, row-major / tiled, us: given
-# M = 2 273.8 / 279.7, M = 3 291.5 / 282.4, M = 7 303.7 / 288.2; per token M = 9 284.8 / 287.1, M = 10
-# 299.2 / 298.0, M = 12 305.2 / 298.7).
+# Split-K GEMVs take the tiled rows earlier where their workgroups share them in LDS (k_gemv_wide32, as
+# krq_gemv_fp8_shares_rows tells): with a given scale from three rows, scaled per token from eleven
+# (QKV, O, gate_up and down of eight layers in one graph, row-major / tiled, us: given M = 2 273.8 /
+# 279.7, M = 3 291.5 / 282.4, M = 7 303.7 / 288.2; per token M = 9 284.8 / 287.1, M = 10 299.2 / 298.0,
+# M = 12 305.2 / 298.7). Launches that do not share them lose by the padding to sixteen rows: one K pass
+# over a whole row (linear_fp8 over a layer's four projections at M = 5 36.4 us row-major, 43.0 tiled),
+# weights without a tiled copy (down, given scale, M = 5 11.3 / 11.8, M = 8 11.7 / 12.0), N = 16 mod 64
+# (2,576 x 9,728, M = 5 8.9 / 9.5) and splits longer than LDS holds (2,560 x 16,384 in two, M = 5 14.2
+# / 16.1). Split-K launches of those kinds take the tiled rows from TILED_MIN_ROWS (M = 11 / 12 per token
+# 9.7 / 9.8 row-major, 10.0 / 10.0 tiled at 2,576 x 9,728), with a given scale from eleven (M = 11 without
+# a tiled copy: QKV 8.8 / 8.4, down 12.3 / 12.1).
 TILED_MIN_ROWS_SPLIT = {"given": 3, "token": 11}
+TILED_MIN_ROWS_SPLIT_APART = {"given": 11, "token": TILED_MIN_ROWS}
+
+
+def _tiled_least(q, M, split, a):
+    """The rows from which a gemv_fp8 call of M rows takes tiled rows."""
+    kind = "token" if a is None else "given"
+    if split == 1 or not TILED_MIN_ROWS_SPLIT[kind] <= M < TILED_MIN_ROWS:
+        return TILED_MIN_ROWS
+    N, K = q[0].shape
+    shared = getattr(q, "tiled", None) is not None and L.lib().krq_gemv_fp8_shares_rows(M, N, K, split, L.W_TILED)
+    return (TILED_MIN_ROWS_SPLIT if shared else TILED_MIN_ROWS_SPLIT_APART)[kind]
 
 
 def _tiled_rows(x, a, xs, algo, least=TILED_MIN_ROWS):
@@ -398,8 +414,7 @@ def gemv_fp8(x, q, split=1, a=None, xs=None, algo=L.ALGO_AUTO):
     mode = L.OUT_BF16 if split == 1 else L.OUT_PARTIAL
     if xs is None and _fits_fused(x, split, a):
         return gemv_fp8_bf16_launch(x, q, split, mode, a, algo)
-    least = TILED_MIN_ROWS if split == 1 else TILED_MIN_ROWS_SPLIT["token" if a is None else "given"]
-    if _tiled_rows(x, a, xs, algo, least):
+    if _tiled_rows(x, a, xs, algo, _tiled_least(q, M, split, a)):
         x8t, s = _tiled_operand(x, a)
         return gemv_fp8_tiled_launch(x8t, s, q, M, split, mode)
     x8, s = _activation_fp8(x, a, xs)

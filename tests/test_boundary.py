@@ -260,3 +260,33 @@ def test_given_scale_rows_keep_the_picked_cast(monkeypatch):
     monkeypatch.setattr(fp8, "_cast", fp8._cast_torch)
     assert not any(fp8._tiled_rows(v, a, None, L.ALGO_AUTO, 3) for v in x.values())
     assert all(fp8._tiled_rows(v, None, None, L.ALGO_AUTO, 3) for v in x.values())
+
+
+def test_tiled_rows_only_where_shared():
+    """Below TILED_MIN_ROWS, tiled rows only for the launches that share them in LDS: tiled weights, N
+    in whole groups of four row blocks, the split's tiles within LDS, one row block per wave; the
+    head's persistent launch on a grid that fills the chip."""
+    lib = L.lib()
+    shares = lib.krq_gemv_fp8_shares_rows
+    assert shares(5, 6144, 2560, 2, L.W_TILED) == shares(16, 2560, 9728, 4, L.W_TILED) == 1
+    assert shares(3, 65536, 1024, 2, L.W_TILED) == 1 and shares(5, 65536, 1024, 2, L.W_TILED) == 0  # (paired above 4 rows)
+    for bad in ((5, 6144, 2560, 2, L.W_ROWMAJOR), (5, 6160, 2560, 2, L.W_TILED), (5, 2560, 16384, 2, L.W_TILED),
+                (5, 6144, 2560, 3, L.W_TILED), (5, 6144, 2592, 2, L.W_TILED), (1, 6144, 2560, 2, L.W_TILED),
+                (17, 6144, 2560, 2, L.W_TILED), (5, 0, 2560, 2, L.W_TILED), (5, 6144, 2560, 0, L.W_TILED)):
+        assert shares(*bad) == 0, bad
+    head = lib.krq_lmhead_shares_rows
+    assert head(5, 151936, 2560, L.W_TILED) == head(16, 32000, 4096, L.W_TILED) == 1
+    for bad in ((5, 151936, 2560, L.W_ROWMAJOR), (5, 152064, 3584, L.W_TILED), (5, 16448, 2560, L.W_TILED),
+                (5, 128256, 8192, L.W_TILED), (1, 151936, 2560, L.W_TILED), (17, 151936, 2560, L.W_TILED),
+                (5, 0, 2560, L.W_TILED), (5, 151936, 0, L.W_TILED), (5, 151936, 2496, L.W_TILED)):
+        assert head(*bad) == 0, bad
+
+    a = fp8.SharedScale(torch.ones(1), torch.ones(()))
+    t = torch.zeros(1)
+    w8 = torch.empty(2560, 9728, device="meta")
+    for scale, least, apart in ((a, 3, 11), (None, 11, 13)):
+        for M in range(1, 33):
+            assert fp8._tiled_least((w8, t), M, 1, scale) == 13
+            for q, want in ((fp8.FP8Weight(w8, t, t), least), (fp8.FP8Weight(w8, t, None), apart), ((w8, t), apart),
+                            (fp8.FP8Weight(w8[:2544], t, t), apart)):
+                assert (M >= fp8._tiled_least(q, M, 4, scale)) == (M >= want)
