@@ -29,8 +29,8 @@ HEADROOM = float(os.environ.get("ENGINE_FP8_HEADROOM", "4"))
 DECODE_MAX_ROWS = 32  # rows handled by one launch of the skinny kernels
 # From this many rows linear_fp8 runs gemm_fp8. Per Qwen3-4B decoder layer (the four projections,
 # weights cold in the caches) against hipBLASLt on MI355X, us: M = 33 39.2 / 39.5, M = 48 40.0 / 43.3,
-# M = 77 44.2 / 46.9, M = 127 46.8 / 51.8, M = 160 54.8 / 54.4, M = 256 58.1 / 67.4, M = 1024 133 / 141;
-# and the library's call takes 20 us of host time where this one takes 8.
+# M = 77 44.2 / 46.9, M = 127 46.8 / 51.8, M = 160 54.8 / 54.4, M = 256 58.1 / 67.4, M = 1024 133 / 141.
+# Which weights it takes below PER_CHANNEL_MIN_ROWS: _ring_pays.
 PREFILL_MIN_ROWS = DECODE_MAX_ROWS + 1
 # The library takes one scale per weight; fewer rows than this keep refusing per-channel ones there.
 PER_CHANNEL_MIN_ROWS = 128
@@ -238,12 +238,13 @@ def _weight_operand(q):
     w8, ws = q[0], q[1]
     tiled = getattr(q, "tiled", None)
     L.require_device(w8, ws)
-    _check_weight_scale(ws, w8.shape[0])
+    shape = w8.shape
+    _check_weight_scale(ws, shape[0])
     if tiled is not None:
-        return tiled, L.W_TILED, ws, w8.shape
+        return tiled, L.W_TILED, ws, shape
     if w8.dtype != torch.float8_e4m3fn or w8.dim() != 2 or not w8.is_contiguous():
         raise ValueError("expected a contiguous float8_e4m3fn [N, K] weight")
-    return w8, L.W_ROWMAJOR, ws, w8.shape
+    return w8, L.W_ROWMAJOR, ws, shape
 
 
 FUSED_MAX_ELEMS = 8 * 64 * 64  # activation slice the GEMV can quantize in its prologue (static scale)
@@ -511,14 +512,16 @@ def linear_fp8(x, q, a=None, amax_out=None):
     None to scale by this tensor's own range (running max kept in amax_out).
     Reference: engine/kernels/fp8.py:97-106. Decode sizes (M <= 32) run the HIP GEMV; more rows
     run this library's GEMM (gemm_fp8) where its e4m3 kernels take the weight (N and K multiples of
-    128, K >= 256); the rest keep the reference's library GEMM, torch._scaled_mm (hipBLASLt on
-    ROCm)."""
+    128, K >= 256) and, below 128 rows, where it pays (_ring_pays); the rest keep the reference's
+    library GEMM, torch._scaled_mm (hipBLASLt on ROCm)."""
     w8, ws = q[0], q[1]
-    if x.dim() == 2 and x.shape[0] > DECODE_MAX_ROWS and _cast is _cast_hip and x.shape[0] >= _gemm_min_rows(w8, ws):
+    M = x.shape[0]
+    gemm = M > DECODE_MAX_ROWS and x.dim() == 2 and _takes_gemm(M, w8, ws)
+    if gemm and _cast is _cast_hip:
         return _linear_gemm(x, q, a, amax_out)
     x8 = None
     if a is None:
-        if x.dim() == 2 and x.shape[0] > DECODE_MAX_ROWS and _cast is _cast_hip:
+        if x.dim() == 2 and M > DECODE_MAX_ROWS and _cast is _cast_hip:
             a, x8 = _act_scale_cast(x)
         else:
             a = ActScale(x)
@@ -527,12 +530,12 @@ def linear_fp8(x, q, a=None, amax_out=None):
     if x8 is None and _fits_fused(x, 1, a):
         return gemv_fp8_bf16_launch(x, q, 1, L.OUT_BF16, a)
     if x8 is None and _tiled_rows(x, a, None, L.ALGO_AUTO):
-        return gemv_fp8_tiled_launch(cast_tiled(x, a), _one(a.scale), q, x.shape[0], 1, L.OUT_BF16)
+        return gemv_fp8_tiled_launch(cast_tiled(x, a), _one(a.scale), q, M, 1, L.OUT_BF16)
     if x8 is None:
         x8 = _cast(x, a)
-    if x.shape[0] <= DECODE_MAX_ROWS:
+    if M <= DECODE_MAX_ROWS:
         return gemv_fp8_launch(x8, _one(a.scale), q, 1, L.OUT_BF16)
-    if x.shape[0] >= _gemm_min_rows(w8, ws):
+    if gemm:
         return gemm_fp8(x8, q, xs=_one(a.scale))
     return torch._scaled_mm(x8, w8.t(), scale_a=a.scale, scale_b=ws, out_dtype=torch.bfloat16)
 
@@ -580,14 +583,43 @@ def _linear_gemm(x, q, a, amax_out):
 def _gemm_min_rows(w8, ws):
     """The rows from which linear_fp8 runs this library's GEMM on a weight. Below
     PER_CHANNEL_MIN_ROWS what the library's product refuses (per-channel scales, scales that are
-    not fp32) or alone takes (a weight that does not start on 16 bytes) stays with it."""
+    not fp32) or alone takes (a weight that does not start on 16 bytes) stays with it; see _ring_pays
+    for the rest."""
     if not _ring_gemm_fits(w8):
         return float("inf")
     own = ws.numel() == 1 and ws.dtype == torch.float32 and w8.data_ptr() % 16 == 0
     return PREFILL_MIN_ROWS if own else PER_CHANNEL_MIN_ROWS
 
 
+def _takes_gemm(M, w8, ws):
+    """Whether linear_fp8 runs this library's GEMM on M > DECODE_MAX_ROWS rows of a weight."""
+    return M >= _gemm_min_rows(w8, ws) and (M >= PER_CHANNEL_MIN_ROWS or _ring_pays(M, *w8.shape))
+
+
+def _ring_pays(M, N, K):
+    """Below PER_CHANNEL_MIN_ROWS rows: the weights on which a linear_fp8 call is no slower through this
+    library's GEMM than through torch._scaled_mm. Such calls are made one by one (prefill), where the
+    library's takes 39 us of host time and this one 16.5, so up to 64 MiB of weights it is the faster
+    one, also where its product is not. Measured, us, called / captured in a graph with others:
+      19,456 x 2,560  M = 77 24.7 against 40.6 / 25.2 against 25.5, M = 127 28.5 against 39.2 / 29.2, 26.5
+      4,096 x 5,120   M = 64 21 against 42 / 21.7 against 16.7
+      1,024 x 6,144   M = 64 18.7 against 42 / 17.0 against 12.5
+      128 x 16,384    M = 64 33 against 42 / 33.2 against 15.1; 128 x 32,768 61 against 43
+    (the last three: few tiles over a long K that the plan does not split, for which a captured call
+    is slower; past K = 16,384 the called one is too). Larger weights keep the library (28,672 x 8,192
+    M = 127 77 against 61, 32,000 x 4,096 51 against 40, 16,384 x 16,384 84 against 76) but for
+    vocabularies over short rows (151,936 x 2,560 M = 77 92 against 114, 65,536 x 3,584 M = 64 50
+    against 50; 80,000 x 4,096 M = 33 98 against 85) and long rows in split K (8,192 x 28,672 M = 77
+    64 against 198, 2,560 x 32,768 42 against 108, 8,192 x 18,432 M = 64 46 against 60). From 2 GiB
+    gemm_fp8 leaves the ring kernels all this was measured on."""
+    if N * K > 1 << 26:
+        return N * K < 0x7fffffff and ((N >= 65536 and K < 4096) or (2560 <= N <= 8192 and K >= 18432))
+    return K <= 16384 or L.lib().krq_gemm_fp8_ws_bytes(L.X_FP8, M, N, K) != 0
+
+
 def _ring_gemm_fits(w8):
     """The weight shapes gemm_fp8 multiplies with its ring kernels on e4m3 rows."""
-    return (w8.dtype == torch.float8_e4m3fn and w8.dim() == 2 and w8.is_contiguous() and w8.shape[0] % 128 == 0
-            and w8.shape[1] % 128 == 0 and w8.shape[1] >= 256)
+    if w8.dtype != torch.float8_e4m3fn or w8.dim() != 2 or not w8.is_contiguous():
+        return False
+    N, K = w8.shape
+    return N % 128 == 0 and K % 128 == 0 and K >= 256

@@ -290,3 +290,26 @@ def test_tiled_rows_only_where_shared():
             for q, want in ((fp8.FP8Weight(w8, t, t), least), (fp8.FP8Weight(w8, t, None), apart), ((w8, t), apart),
                             (fp8.FP8Weight(w8[:2544], t, t), apart)):
                 assert (M >= fp8._tiled_least(q, M, 4, scale)) == (M >= want)
+
+
+def test_linear_gemm_weights(monkeypatch):
+    """linear_fp8 at 33 to 127 rows takes its own GEMM up to 64 MiB of weights (past K = 16,384 in split
+    K), beyond that for long vocabularies over short rows and for long rows, never from 2 GiB; from
+    128 rows always."""
+    class Plan:
+        def __init__(self, split):
+            self.krq_gemm_fp8_ws_bytes = lambda kind, M, N, K: 1024 if split else 0
+
+    for split in (False, True):
+        monkeypatch.setattr(L, "lib", lambda: Plan(split))
+        for M in (33, 64, 65, 127):
+            for N, K in ((128, 256), (2560, 4096), (19456, 2560), (16384, 4096), (4096, 5120), (128, 16384),
+                         (151936, 2560), (65536, 3584), (8192, 28672), (2560, 32768)):
+                assert fp8._ring_pays(M, N, K), (M, N, K)
+            for N, K in ((28672, 8192), (32000, 4096), (16384, 16384), (80000, 4096), (2048, 65536), (51200, 5120),
+                         (1 << 20, 2048), (1 << 21, 1024)):
+                assert not fp8._ring_pays(M, N, K), (M, N, K)
+            assert fp8._ring_pays(M, 128, 32768) == fp8._ring_pays(M, 2048, 32768) == split
+    w8 = torch.empty(1, 1, device="meta", dtype=torch.float8_e4m3fn).expand(28672, 8192)
+    monkeypatch.setattr(fp8, "_gemm_min_rows", lambda w, ws: fp8.PREFILL_MIN_ROWS)
+    assert not fp8._takes_gemm(127, w8, None) and fp8._takes_gemm(128, w8, None)
