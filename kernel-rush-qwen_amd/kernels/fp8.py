@@ -229,9 +229,11 @@ def pick_cast(log):
 # skinny GEMM / GEMV
 # ---------------------------------------------------------------------------------------------
 def _check_weight_scale(ws, N):
-    """The kernels read a weight's scale as one fp32 value or one per output row."""
-    if ws.dtype != torch.float32 or ws.numel() not in (1, N) or not ws.is_contiguous():
+    """The kernels read a weight's scale as one fp32 value or one per output row; 1 for the latter."""
+    n = ws.numel()
+    if ws.dtype != torch.float32 or (n != 1 and (n != N or not ws.is_contiguous())):
         raise ValueError(f"weight scale must be contiguous fp32 with 1 or {N} values, got {ws.dtype} {tuple(ws.shape)}")
+    return 1 if n > 1 else 0
 
 
 def _weight_operand(q):
@@ -312,13 +314,12 @@ def _one(scale):
     return scale if scale.numel() == 1 else scale.reshape(1)
 
 
-def _fits_fused(x, split, a):
+def _fits_fused(x, M, K, split, a):
     """One row quantized in the GEMV's prologue (its activation wave). More rows with a given
     scale are cast first (row-major, or tiled from TILED_MIN_ROWS): quantizing them in the prologue
     measured slower on MI355X at every M > 1 (split 1, us, prologue / cast + GEMV): QKV M = 4
     9.19 / 6.92, M = 8 10.62 / 7.19; gate_up M = 4 15.78 / 11.33, M = 8 23.66 / 11.90."""
-    M, K = x.shape
-    if x.dtype != torch.bfloat16 or M != 1 or K % 64:
+    if M != 1 or K % 64 or x.dtype != torch.bfloat16:
         return False
     if a is None:
         return K <= FUSED_MAX_ELEMS_DYN
@@ -363,26 +364,24 @@ TILED_MIN_ROWS_SPLIT_APART = {"given": 11, "token": TILED_MIN_ROWS}
 
 
 def _tiled_least(q, M, split, a):
-    """The rows from which a gemv_fp8 call of M rows takes tiled rows."""
+    """The rows from which a split-K gemv_fp8 call of M < TILED_MIN_ROWS rows takes tiled rows."""
     kind = "token" if a is None else "given"
-    if split == 1 or not TILED_MIN_ROWS_SPLIT[kind] <= M < TILED_MIN_ROWS:
+    if M < TILED_MIN_ROWS_SPLIT[kind]:
         return TILED_MIN_ROWS
     N, K = q[0].shape
     shared = getattr(q, "tiled", None) is not None and L.lib().krq_gemv_fp8_shares_rows(M, N, K, split, L.W_TILED)
     return (TILED_MIN_ROWS_SPLIT if shared else TILED_MIN_ROWS_SPLIT_APART)[kind]
 
 
-def _tiled_rows(x, a, xs, algo, least=TILED_MIN_ROWS):
+def _tiled_rows(x, M, K, a, xs, algo, least=TILED_MIN_ROWS):
     """bf16 rows at `least` <= M <= 32 go through quant_rows_tiled (scaled per token) or
     cast_tiled (a given scale) and the GEMV on tiled activations (the operands of quant_rows / _cast
     + the row-major e4m3 GEMV, with contiguous loads); fewer rows, rows longer than the tiled
     kernels take, and below TILED_MIN_ROWS rows that do not start on 16 bytes (the row-major
     quantizers take any address) use the row-major kernels, as do given-scale rows where pick_cast
     has put torch's cast in the place of the HIP one."""
-    M, K = x.shape
-    return (xs is None and x.dtype == torch.bfloat16 and least <= M <= DECODE_MAX_ROWS
-            and K % 64 == 0 and K <= TILED_ROWS_MAX_K and algo != L.ALGO_VALU
-            and (a is None or _cast is _cast_hip)
+    return (least <= M <= DECODE_MAX_ROWS and xs is None and x.dtype == torch.bfloat16 and K % 64 == 0
+            and K <= TILED_ROWS_MAX_K and algo != L.ALGO_VALU and (a is None or _cast is _cast_hip)
             and (M >= TILED_MIN_ROWS or x.data_ptr() % 16 == 0))
 
 
@@ -413,9 +412,10 @@ def gemv_fp8(x, q, split=1, a=None, xs=None, algo=L.ALGO_AUTO):
     M, K = x.shape
     assert K % split == 0
     mode = L.OUT_BF16 if split == 1 else L.OUT_PARTIAL
-    if xs is None and _fits_fused(x, split, a):
+    if xs is None and _fits_fused(x, M, K, split, a):
         return gemv_fp8_bf16_launch(x, q, split, mode, a, algo)
-    if _tiled_rows(x, a, xs, algo, _tiled_least(q, M, split, a)):
+    least = TILED_MIN_ROWS if split == 1 or M >= TILED_MIN_ROWS else _tiled_least(q, M, split, a)
+    if _tiled_rows(x, M, K, a, xs, algo, least):
         x8t, s = _tiled_operand(x, a)
         return gemv_fp8_tiled_launch(x8t, s, q, M, split, mode)
     x8, s = _activation_fp8(x, a, xs)
@@ -426,11 +426,12 @@ def gemv_swiglu_fp8(x, q, a=None, xs=None, algo=L.ALGO_AUTO):
     """FP8 counterpart of kernels.gemv.gemv_swiglu: q quantizes w_gu [2I, K] = [gate; up];
     returns bf16(bf16(silu(bf16 g)) * bf16 u) [M, I]. Called as fp8.gemv_swiglu_fp8(x, q) by the
     reference's experiments/modal_fp8.py:67."""
-    if xs is None and _fits_fused(x, 1, a):
+    M, K = x.shape
+    if xs is None and _fits_fused(x, M, K, 1, a):
         return gemv_fp8_bf16_launch(x, q, 1, L.OUT_SWIGLU, a, algo)
-    if _tiled_rows(x, a, xs, algo):
+    if _tiled_rows(x, M, K, a, xs, algo):
         x8t, s = _tiled_operand(x, a)
-        return gemv_fp8_tiled_launch(x8t, s, q, x.shape[0], 1, L.OUT_SWIGLU)
+        return gemv_fp8_tiled_launch(x8t, s, q, M, 1, L.OUT_SWIGLU)
     x8, s = _activation_fp8(x, a, xs)
     return _chunked(x8, s, lambda xc, sc: gemv_fp8_launch(xc, sc, q, 1, L.OUT_SWIGLU, algo))
 
@@ -445,15 +446,15 @@ def swiglu_cast_fp8(x, q, out_a, a=None, xs=None):
     [16 ceil(M / 16) * I], scale fp32 [1]) for gemv_fp8_tiled_launch."""
     w, layout, ws, (N, K) = _weight_operand(q)
     M = x.shape[0]
-    if M > DECODE_MAX_ROWS or x.shape[1] != K:
+    if M > DECODE_MAX_ROWS or x.dim() != 2 or x.shape[1] != K:
         raise ValueError(f"swiglu_cast_fp8: x {tuple(x.shape)} against w [{N}, {K}] (M <= {DECODE_MAX_ROWS})")
     if N % 128:
         raise ValueError(f"swiglu_cast_fp8: the activation width {N // 2} must be a multiple of 64")
-    if xs is None and _fits_fused(x, 1, a):
+    if xs is None and _fits_fused(x, M, K, 1, a):
         xin = _rows(x)
         kind, x_scale, x_inv = (L.X_BF16_DYN, None, None) if a is None else \
             (L.X_BF16_STATIC, _one(a.scale), _one(a.inv))
-    elif _tiled_rows(x, a, xs, L.ALGO_AUTO):
+    elif _tiled_rows(x, M, K, a, xs, L.ALGO_AUTO):
         xin, x_scale = _tiled_operand(x, a)
         kind, x_inv = L.X_FP8_TILED, None
     else:
@@ -515,21 +516,21 @@ def linear_fp8(x, q, a=None, amax_out=None):
     128, K >= 256) and, below 128 rows, where it pays (_ring_pays); the rest keep the reference's
     library GEMM, torch._scaled_mm (hipBLASLt on ROCm)."""
     w8, ws = q[0], q[1]
-    M = x.shape[0]
-    gemm = M > DECODE_MAX_ROWS and x.dim() == 2 and _takes_gemm(M, w8, ws)
+    M, K = x.shape
+    gemm = M > DECODE_MAX_ROWS and _takes_gemm(M, w8, ws)
     if gemm and _cast is _cast_hip:
         return _linear_gemm(x, q, a, amax_out)
     x8 = None
     if a is None:
-        if x.dim() == 2 and M > DECODE_MAX_ROWS and _cast is _cast_hip:
+        if M > DECODE_MAX_ROWS and _cast is _cast_hip:
             a, x8 = _act_scale_cast(x)
         else:
             a = ActScale(x)
         if amax_out is not None:
             amax_out.copy_(torch.maximum(amax_out, a.amax.reshape(1)))
-    if x8 is None and _fits_fused(x, 1, a):
+    if x8 is None and _fits_fused(x, M, K, 1, a):
         return gemv_fp8_bf16_launch(x, q, 1, L.OUT_BF16, a)
-    if x8 is None and _tiled_rows(x, a, None, L.ALGO_AUTO):
+    if x8 is None and _tiled_rows(x, M, K, a, None, L.ALGO_AUTO):
         return gemv_fp8_tiled_launch(cast_tiled(x, a), _one(a.scale), q, M, 1, L.OUT_BF16)
     if x8 is None:
         x8 = _cast(x, a)
@@ -547,14 +548,14 @@ def _linear_gemm(x, q, a, amax_out):
     through ActScale and gemm_fp8, 20 us this way."""
     w8, ws = q[0], q[1]
     N, K = w8.shape
-    _check_weight_scale(ws, N)
+    wpr = _check_weight_scale(ws, N)
     if a is not None:
         inv, given = _one(a.inv), _one(a.scale)
         L.require_device(inv, given)
     x2 = _rows(x)
-    M = x2.shape[0]
+    M, kx = x2.shape
     L.require_device(w8, ws)
-    if x2.shape[1] != K:
+    if kx != K:
         raise ValueError(f"x {tuple(x.shape)} does not match w8 {tuple(w8.shape)}")
     lib = L.lib()
     parts = 4 * lib.krq_act_scale_ws_floats(M, K) if a is None else 0
@@ -575,8 +576,8 @@ def _linear_gemm(x, q, a, amax_out):
     else:
         scale = L.ptr(given)
         L.call("krq_cast_fp8", L.ptr(x2), M, K, L.ptr(inv), 0, p + at8, st)
-    L.call("krq_gemm_fp8_ws", p + at8, L.X_FP8, scale, None, 0, L.ptr(w8), L.ptr(ws), 1 if ws.numel() > 1 else 0,
-           M, N, K, p + at_split if split_bytes else None, split_bytes, L.ptr(out), st)
+    L.call("krq_gemm_fp8_ws", p + at8, L.X_FP8, scale, None, 0, L.ptr(w8), L.ptr(ws), wpr, M, N, K,
+           p + at_split if split_bytes else None, split_bytes, L.ptr(out), st)
     return out
 
 

