@@ -25,6 +25,8 @@
 
 #include <stdlib.h>
 
+#include <type_traits>
+
 using namespace krq;
 
 namespace {
@@ -156,7 +158,8 @@ __global__ __launch_bounds__(kMaxNT) void k_gemv_fused(const uint8_t* __restrict
   }
 
   // ---- main loop: operands from the staged slice ----
-  auto consume_slot = [&](int u, int cc) {
+  // (last: as in gemv_bf16.hip; a normalized row with an infinity is NaN as it is)
+  auto consume_slot = [&](auto last, int u, int cc) {
     const int j = jcount > 0 ? wave + min(cc, jcount - 1) * nw : 0;
     const bool ok = cc < jcount, hi = ok && (2 * j + 1 < kts);
     const uint4 bl = sel4(ok, wl[u]), bh = sel4(hi, wh[u]);
@@ -169,8 +172,9 @@ __global__ __launch_bounds__(kMaxNT) void k_gemv_fused(const uint8_t* __restrict
         al[mt] = *reinterpret_cast<const uint4*>(hr + (2 * j) * 64);
         ah[mt] = sel4(2 * j + 1 < kts, *reinterpret_cast<const uint4*>(hr + min(2 * j + 1, kts - 1) * 64));
       } else {
-        al[mt] = xl[u][mt];
-        ah[mt] = xh[u][mt];
+        constexpr bool LAST = decltype(last)::value;
+        al[mt] = LAST ? sel4(ok, xl[u][mt]) : xl[u][mt];
+        ah[mt] = LAST ? sel4(hi, xh[u][mt]) : xh[u][mt];
       }
     }
     if (ALGO == 2) {
@@ -200,12 +204,12 @@ __global__ __launch_bounds__(kMaxNT) void k_gemv_fused(const uint8_t* __restrict
   for (; base + U < jcount; base += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      consume_slot(u, base + u);
+      consume_slot(std::false_type{}, u, base + u);
       load_slot(u, base + u + U);
     }
   }
 #pragma unroll
-  for (int u = 0; u < U; ++u) consume_slot(u, base + u);
+  for (int u = 0; u < U; ++u) consume_slot(std::true_type{}, u, base + u);
   if (ALGO == 2) {
     float a = s0 + s1, au = q0 + q1;
     a += __shfl_xor(a, 16, kWave);

@@ -7,6 +7,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 using namespace krq;
 
@@ -124,25 +125,39 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
     load_w(u, cc);
     load_x(u, cc);
   };
-  auto consume_slot = [&](int u, int cc) {
-    const int j = jcount > 0 ? wave + min(cc, jcount - 1) * nw : 0;
-    const bool ok = cc < jcount, hi = ok && (2 * j + 1 < kts);
+  // LAST: the step may be past this wave's last one, or the split's half step (one tile of two). On the
+  // vector ALUs what is not there is skipped (four layers row-major at M = 1 183.0 us, 188.7 masked);
+  // on the matrix cores, which ignore the execution mask, the activations are zeroed with the
+  // weights, since an infinite one times zero is NaN.
+  const int jlast = __builtin_amdgcn_readfirstlane(jcount), wv = __builtin_amdgcn_readfirstlane(wave);
+  auto consume_slot = [&](auto last, int u, int cc) {
+    constexpr bool LAST = decltype(last)::value, SKIP = LAST && ALGO == 2;
+    const int cs = __builtin_amdgcn_readfirstlane(cc);
+    if (SKIP && cs >= jlast) return;
+    const int j = SKIP ? wv + cs * nw : jcount > 0 ? wave + min(cc, jcount - 1) * nw : 0;
+    const bool ok = SKIP || cc < jcount, hi = ok && (2 * j + 1 < kts);
     uint4 al[MT], ah[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       al[mt] = xl[u][mt];
       ah[mt] = xh[u][mt];
       if constexpr (XL) lines_to_tiles(xl[u][mt], XO ? xl[u][mt] : xh[u][mt], &al[mt], &ah[mt]);
+      if constexpr (LAST && !SKIP) {
+        al[mt] = sel4(ok, al[mt]);
+        ah[mt] = sel4(hi, ah[mt]);
+      }
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       uint4 bl = wl[p][u], bh = wh[p][u];
       if constexpr (RM) lines_to_tiles(wl[p][u], wh[p][u], &bl, &bh);
-      bl = sel4(ok, bl);
-      bh = sel4(hi, bh);
+      if constexpr (!SKIP) {
+        bl = sel4(ok, bl);
+        bh = sel4(hi, bh);
+      }
       if (ALGO == 2) {
         sv[p][0] = dot8_bf16(bl, al[0], sv[p][0]);
-        sv[p][1] = dot8_bf16(bh, ah[0], sv[p][1]);
+        if (!SKIP || hi) sv[p][1] = dot8_bf16(bh, ah[0], sv[p][1]);
       } else {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
@@ -173,7 +188,7 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
     // entered with them in that order waits for every load on its first pass.
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      consume_slot(u, u);
+      consume_slot(std::true_type{}, u, u);
       load_slot(u, u + U);
     }
     base = U;
@@ -188,13 +203,21 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
   for (; base + U < jcount; base += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      consume_slot(u, base + u);
+      consume_slot(std::false_type{}, u, base + u);
       load_slot(u, base + u + U);
       if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
     }
   }
+  // (a last batch of U whole steps needs none of it: a scalar branch, and the shapes of the projections
+  // pay nothing for the others)
+  const int bs = __builtin_amdgcn_readfirstlane(base);
+  if (ALGO != 2 && bs + U == jlast && (kts & 1) == 0) {
 #pragma unroll
-  for (int u = 0; u < U; ++u) consume_slot(u, base + u);
+    for (int u = 0; u < U; ++u) consume_slot(std::false_type{}, u, bs + u);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) consume_slot(std::true_type{}, u, bs + u);
+  }
   if (ALGO == 2) {
     // the four lanes of row r (g = 0..3) hold partial sums of disjoint k: add them; lanes 0..15
     // then carry columns 16 rb + lane in MFMA slot (mt 0, i 0), i.e. output row m = 0
@@ -318,7 +341,7 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* 
     for (int q = 0; q < NS; ++q)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[p][q][mt] = v4f{0.f, 0.f, 0.f, 0.f};
-  auto consume = [&](int u, int j) {
+  auto consume = [&](auto last, int u, int j) {  // (last: as in gemv_bf16_body)
     const bool hi = 2 * j + 1 < kts;
     uint4 al[MT], ah[MT];
 #pragma unroll
@@ -327,6 +350,7 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* 
       const uint8_t* xr = xt + (j * hv + h) * 1024 + 16 * (r & 7);
       al[mt] = *reinterpret_cast<const uint4*>(xr + 128 * (g ^ (h & 1)));
       ah[mt] = *reinterpret_cast<const uint4*>(xr + 128 * ((g + 4) ^ (h & 1)));
+      if constexpr (decltype(last)::value) ah[mt] = sel4(hi, ah[mt]);
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
@@ -345,14 +369,19 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* 
   for (; base + U < nsteps; base += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      consume(u, base + u);
+      consume(std::false_type{}, u, base + u);
       load_slot(u, base + u + U);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  if (base + U == nsteps && (kts & 1) == 0) {  // (whole steps, as in gemv_bf16_body)
 #pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (base + u < nsteps) consume(u, base + u);  // (not zeroed weights: an infinite activation times them is NaN)
+    for (int u = 0; u < U; ++u) consume(std::false_type{}, u, base + u);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (base + u < nsteps) consume(std::true_type{}, u, base + u);
+  }
 
   // element i of lane l: row 16 mt + 4 (l / 16) + i, column 16 rb + l % 16
   const int64_t n = rb * 16 + r;
@@ -457,7 +486,7 @@ __global__ __launch_bounds__(512) void k_gemv_bf16_rows(const uint8_t* __restric
       accu[mt] = v4f{0.f, 0.f, 0.f, 0.f};
     }
     uint4 wl[U], wh[U], ul[U], uh[U], xl[U][MT], xh[U][MT];
-    // every slot load is issued (a slot past the last step reloads it and is masked where consumed)
+    // every slot load is issued (a slot past the last step reloads it and is zeroed where consumed)
     auto load_slot = [&](int u, int cc) {
       const int j = min(cc, nsteps - 1);
       const int64_t t0 = 2 * j, t1 = (2 * j + 1 < kts) ? t0 + 1 : t0;
@@ -473,10 +502,17 @@ __global__ __launch_bounds__(512) void k_gemv_bf16_rows(const uint8_t* __restric
         xh[u][mt] = ld16(xr[mt] + t1 * 64);
       }
     };
-    auto consume_slot = [&](int u, int cc) {
+    auto consume_slot = [&](auto last, int u, int cc) {  // (last: as in gemv_bf16_body)
       const int j = min(cc, nsteps - 1);
       const bool ok = cc < nsteps, hi = ok && (2 * j + 1 < kts);
       const uint4 bl = sel4(ok, wl[u]), bh = sel4(hi, wh[u]);
+      if constexpr (decltype(last)::value) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          xl[u][mt] = sel4(ok, xl[u][mt]);
+          xh[u][mt] = sel4(hi, xh[u][mt]);
+        }
+      }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_v8bf(xl[u][mt]), as_v8bf(bl), acc[mt], 0, 0, 0);
@@ -498,12 +534,12 @@ __global__ __launch_bounds__(512) void k_gemv_bf16_rows(const uint8_t* __restric
     for (; base + U < nsteps; base += U) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        consume_slot(u, base + u);
+        consume_slot(std::false_type{}, u, base + u);
         load_slot(u, base + u + U);
       }
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) consume_slot(u, base + u);
+    for (int u = 0; u < U; ++u) consume_slot(std::true_type{}, u, base + u);
     // lane (g, r), element i of tile mt: output row m = 16 mt + 4 g + i, column n0 + r
     const int64_t n = n0 + r;
     if (n < r1) {

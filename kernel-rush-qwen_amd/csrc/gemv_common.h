@@ -123,7 +123,7 @@ KRQ_DEV const uint8_t* w_addr(const uint8_t* w, int64_t rb, int64_t t, int64_t r
 // lines_to_tiles then gives every lane the bytes w_addr would have: lanes c and c ^ 8 exchange one
 // 16-byte register each (lanes 8-15 take the second load's low half of the line, lanes 0-7 the first
 // load's high half), one DPP move per dword. half: the step holds its low tile only (the high
-// chunks repeat the low ones; the consumer masks them).
+// chunks repeat the low ones and are not consumed).
 // Measured on row-major bf16 weights (four Qwen3-4B layers in one graph; on tiled copies of them 174
 // us at M = 1 and 215 at M = 16): M = 1 238.6 -> 187.0 us, M = 16 293.5 -> 237.4, M = 32 398 -> 337.
 // The activation rows of the matrix-core kernels are read the same way: M = 32 361 -> 337, and with

@@ -316,3 +316,62 @@ def test_bf16_infinity_in_the_last_step(dev, M, steps):
     y = gemv(x.to(dev), w.to(dev), 1).float().cpu()
     assert torch.equal(y[M - 1], torch.full((8192,), float("inf")) * torch.sign(w[:, -1].float()))
     assert torch.isfinite(y[:M - 1]).all()
+
+
+# The same where the last step of K (or of a split) holds one tile of two (K / split an odd multiple of 32)
+# and where waves have fewer steps than slots, on every BF16 launch: one row, few rows, 16-column and wide
+# blocks (N = 16 and 0 mod 64 on at least half the compute units), two row tiles, both weight layouts,
+# SwiGLU (mixed launch up to 16 rows), the row partition and the fused GEMV.
+@pytest.mark.parametrize("M", [1, 3, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K,split", [(8192, 32, 1), (8208, 32 * 9, 1), (8192, 32 * 9, 1), (2048, 4 * 32 * 11, 4),
+                                       (8256, 32 * 17, 1), (8256, 64 * 5, 1), (144, 32 * 7, 1), (144, 64 * 3, 1)])
+def test_bf16_infinity_in_a_half_step(dev, M, N, K, split):
+    from kernels import fused_gemv as FG, gemv as G
+    g = torch.Generator().manual_seed(98)
+    w = (torch.randn(2 * N, K, generator=g) * 0.02).to(torch.bfloat16)
+    w[:, -1] = torch.where(w[:, -1] == 0, 0.01, w[:, -1].float()).to(torch.bfloat16)
+    w[:N, -1] = w[:N, -1].abs()  # (gates of plus infinity: the SwiGLU is the up product's infinity)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    x[M - 1, -1] = float("inf")
+    xd, up, both = x.to(dev), w[N:].contiguous().to(dev), w.to(dev)
+    want = torch.full((N,), float("inf")) * torch.sign(w[N:, -1].float())
+
+    def check(y):
+        y = y.float().cpu()
+        last = y[-1] if y.dim() == 3 else y  # (the last split holds the infinity)
+        assert torch.equal(last[M - 1], want)
+        assert torch.isfinite(last[:M - 1]).all() and (y.dim() == 2 or torch.isfinite(y[:-1]).all())
+
+    for _ in range(2):  # row-major, then packed
+        check(G.gemv(xd, up, split))
+        check(FG.gemv_fused(xd, up, split))
+        check(FG.gemv_swiglu_fused(xd, both))
+        check(G.gemv_swiglu(xd, both))
+        if split == 1:
+            check(G.gemv_rows(xd, up, 60))
+            check(G.gemv_rows(xd, both, 60, swiglu=True))
+        G.pack(up)
+        G.pack(both)
+
+
+@pytest.mark.parametrize("M", [1, 4, 16, 32])
+def test_bf16_infinity_in_chained_down(dev, M):
+    """The chained MLP's down stage on an infinite activation: the two launches' partials."""
+    from kernels import gemv as G
+    from kernels.mlp import PersistentMLP
+    H, I, S = 512, 4 * 64 * 5, 4
+    g = torch.Generator().manual_seed(99)
+    x = torch.randn(M, H, generator=g).to(torch.bfloat16).abs()
+    gu = (torch.randn(2 * I, H, generator=g) * 0.02).to(torch.bfloat16)
+    gu[I - 1], gu[-1] = 3e37, 3e37  # act's last column overflows, the other columns are finite
+    down = (torch.randn(H, I, generator=g) * 0.02).to(torch.bfloat16)
+    down[:, -1] = torch.where(down[:, -1] == 0, 0.01, down[:, -1].float()).to(torch.bfloat16)
+    xd, gud, dd = x.to(dev), gu.to(dev), down.to(dev)
+    act = G.gemv_swiglu(xd, gud)
+    assert torch.isinf(act[:, -1]).all() and torch.isfinite(act[:, :-1]).all()
+    want = torch.full((M, H), float("inf")) * torch.sign(down[:, -1].float())
+    part = G.gemv(act, dd, S)
+    assert torch.equal(part[-1].cpu(), want) and torch.isfinite(part[:-1]).all()
+    mlp = PersistentMLP(M, H, I, dev, split=S, chunk=64, chained=True)
+    got = mlp(xd, gud, dd)
+    assert torch.equal(mlp.act, act) and torch.equal(got, part) and not mlp.failed()
