@@ -628,15 +628,15 @@ bool launch_swiglu_mixed(int layout, int M, int64_t NO, int nw, size_t smem, hip
 // k_gemv_bf16_wide where it applies (false otherwise): launches of more than four rows whose replaced
 // plan has two waves, whole groups of four row blocks on at least half the compute units, the split's
 // activation rows within LDS. Four Qwen3-4B layers in one graph, us, 16-column blocks / wide, row-major
-// weights: M = 3 194.1 / 195.5 and M = 4 199.1 / 197.6 (left narrow), M = 6 202 / 190, M = 16 246 / 221, M = 32 336 / 256; packed: M = 16 205 / 189,
-// M = 32 291 / 229. Four slots: two measured 254 at M = 16 row-major, six 228, eight 234. The two-matrix
+// weights: M = 3 194.1 / 195.5 and M = 4 199.1 / 197.6 (left narrow), M = 6 202 / 190, M = 16 246 / 221,
+// M = 32 336 / 256; packed: M = 16 205 / 189, M = 32 291 / 229. Four slots: two measured 254 at M = 16 row-major, six 228, eight 234. The two-matrix
 // SwiGLU block (152 workgroups for gate_up) is wide above 16 rows only: at M = 16 23.8 us against
 // 25.2 wide, at M = 32 34.0 against 21.
 bool launch_wide(int layout, int M, int mode, int pb, int nw, int64_t NO, int split, hipStream_t s, const uint8_t* x,
                  const uint8_t* w, int64_t K, int kts, void* out) {
   const int64_t groups = NO / 16 / kWideRb;
   const int kib = (kts + 1) / 2 * ((M + 7) / 8);  // LDS for the split's activation rows
-  if (M <= 4 || pb != 1 || nw != 2 || (NO / 16) % kWideRb != 0 || groups * split < 128 || kib > 160)
+  if (M <= 4 || pb != 1 || nw != 2 || (NO / 16) % kWideRb != 0 || 2 * groups * split < kCUs || kib > 160)
     return false;
   if (M * 2 * K > 0x7fffffff) return false;  // (32-bit activation offsets)
   const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(split)), block(kWideRb * 64);
