@@ -250,3 +250,47 @@ def test_scales_refused(dev, M):
     for s in (F.SharedScale(a.inv.double(), a.scale), F.SharedScale(a.inv, a.scale.double())):
         with pytest.raises((RuntimeError, ValueError)):
             F.linear_fp8(x, q, s)
+
+
+@pytest.mark.parametrize("given", [False, True])
+@pytest.mark.parametrize("M,N,K", [(77, 384, 512), (40, 2560, 9728), (256, 2560, 9728)])
+def test_linear_fp8_capture_and_streams(dev, M, N, K, given):
+    """linear_fp8's one-allocation route (scale, e4m3 rows and split-K partials in one workspace freed at
+    return) captured in a graph, with the running maximum: every replay on new inputs, eager calls on
+    the same shapes in between, equals the eager result; and on two side streams whose calls overlap."""
+    q = F.quantize_weight(bf((N, K), 61, 0.02).to(dev))
+    xs = [bf((M, K), 62 + i, 1.0 + i).to(dev) for i in range(4)]
+    a = F.ActScale(xs[3]) if given else None
+    want = [F.linear_fp8(x, q, a) for x in xs]
+    amax = [x.float().abs().amax().clamp_min(1e-6) for x in xs]
+    torch.cuda.synchronize()
+
+    buf, top = xs[0].clone(), torch.zeros(1, device=dev)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = F.linear_fp8(buf, q, a, amax_out=top)
+    for i in (0, 2, 1, 3):
+        buf.copy_(xs[i])
+        top.zero_()
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want[i]), f"replay on input {i}"
+        assert given or top.item() == amax[i].item()
+        assert torch.equal(F.linear_fp8(xs[(i + 1) % 4], q, a), want[(i + 1) % 4])
+
+    here = torch.cuda.current_stream()
+    sides = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got = [[], []]
+    for s in sides:
+        s.wait_stream(here)
+    for r in range(8):  # (workspaces come and go on each stream while the other's are in use)
+        for k, s in enumerate(sides):
+            with torch.cuda.stream(s):
+                got[k].append(F.linear_fp8(xs[(r + k) % 4], q, a))
+    for s in sides:
+        here.wait_stream(s)
+    torch.cuda.synchronize()
+    for k in range(2):
+        for r in range(8):
+            assert torch.equal(got[k][r], want[(r + k) % 4]), (k, r)

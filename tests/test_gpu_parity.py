@@ -657,9 +657,9 @@ def test_cast_tiled(dev, M, K):
 @pytest.mark.parametrize("M", [4, 12, 13, 16, 23])
 def test_static_scale_multi_row_routes(dev, M):
     """A given scale at 1 < M <= 32 (the engine's FP8 decode, engine/engine.py:977-981): linear_fp8,
-    gemv_fp8 (partials) and gemv_swiglu_fp8 cast the rows first - row-major below TILED_MIN_ROWS,
-    tiled (cast_tiled) from there - and run that GEMV: the same bits as those launches called
-    directly, within the bar of the oracle."""
+    gemv_fp8 (partials) and gemv_swiglu_fp8 cast the rows first, row-major or tiled (cast_tiled) by
+    their own lines, and run that GEMV: the same bits as direct launches on row-major rows below
+    TILED_MIN_ROWS and on tiled ones from there, within the bar of the oracle."""
     a = fp8.SharedScale(torch.tensor([448.0 / 5.0], device=dev), torch.tensor(5.0 / 448.0, device=dev))
     sc = a.scale.reshape(1)
 
