@@ -138,7 +138,7 @@ def static_mlp(torch, fp8, dev, M):
 def prefill_times(torch, fp8, M, lin=True):
     """FP8 prefill GEMM at the four Qwen3-4B projections, M rows: krq_gemm_fp8 on e4m3 activations
     against torch._scaled_mm (hipBLASLt) on the same operands, and (lin) the whole linear_fp8
-    (ActScale + cast + this GEMM from 128 rows, the library GEMM below). Returns name -> (us ours,
+    (ActScale + cast + this GEMM from 33 rows; up to 32 rows the GEMV). Returns name -> (us ours,
     us library, us linear_fp8 or None, flops), each the minimum over replays of a graph of 20."""
     dev = torch.device("cuda:0")
     torch.cuda.set_device(dev)

@@ -152,7 +152,8 @@ def quant_rows_tiled(x):
 
 def cast_tiled(x, a):
     """_cast(x, a) in the tiled activation layout of quant_rows_tiled (krq_cast_fp8_tiled): the
-    static- or per-call-scale rows for the GEMV on X_FP8_TILED (from TILED_MIN_ROWS to 32 rows).
+    static- or per-call-scale rows for the GEMV on X_FP8_TILED (up to 32 rows; from how many it pays:
+    TILED_MIN_ROWS and the lines beside it).
     Returns uint8 [16 * ceil(M / 16) * K]; the bytes are _cast's, permuted, pad rows zero."""
     x2 = _rows(x)
     M, K = x2.shape
