@@ -27,10 +27,12 @@ from . import _lib as L
 FP8_MAX = 448.0
 HEADROOM = float(os.environ.get("ENGINE_FP8_HEADROOM", "4"))
 DECODE_MAX_ROWS = 32  # rows handled by one launch of the skinny kernels
-# From this many rows linear_fp8 runs gemm_fp8. Per Qwen3-4B decoder layer (the four projections,
-# weights cold in the caches) against hipBLASLt on MI355X, us: M = 33 39.2 / 39.5, M = 48 40.0 / 43.3,
-# M = 77 44.2 / 46.9, M = 127 46.8 / 51.8, M = 160 54.8 / 54.4, M = 256 58.1 / 67.4, M = 1024 133 / 141.
-# Which weights it takes below PER_CHANNEL_MIN_ROWS: _ring_pays.
+# From this many rows linear_fp8 runs gemm_fp8. Per Qwen3-4B decoder layer (the four projections' products,
+# weights cold in the caches) against hipBLASLt on MI355X, us: M = 33 44.6 / 46.1, M = 48 46.1 / 52.5,
+# M = 77 52.1 / 53.1, M = 96 54.3 / 50.9, M = 127 58.4 / 60.4, M = 128 58.6 / 71.7, M = 160 64.8 / 62.3,
+# M = 256 73.4 / 75.7, M = 512 97.6 / 95.4, M = 1024 157.6 / 152.3, M = 2048 231 / 230, M = 4096 380 / 358.
+# The whole call is faster where it is short (_ring_pays, which also says on which weights it is taken
+# below PER_CHANNEL_MIN_ROWS).
 PREFILL_MIN_ROWS = DECODE_MAX_ROWS + 1
 # The library takes one scale per weight; fewer rows than this keep refusing per-channel ones there.
 PER_CHANNEL_MIN_ROWS = 128
@@ -546,7 +548,7 @@ def _linear_gemm(x, q, a, amax_out):
     """linear_fp8 on the ring GEMM: the scale (without a given one), the cast and the product, their
     scale, e4m3 rows and partials in one allocation beside the output. A call on a short prompt is
     host work (the launches take 3 us each): 37 us with an allocation per piece and the launches
-    through ActScale and gemm_fp8, 20 us this way."""
+    through ActScale and gemm_fp8, 17 us this way."""
     w8, ws = q[0], q[1]
     N, K = w8.shape
     wpr = _check_weight_scale(ws, N)
