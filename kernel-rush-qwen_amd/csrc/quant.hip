@@ -8,6 +8,7 @@
 #include <stdio.h>
 
 #include <stdlib.h>
+#include <algorithm>
 #include "gemv_common.h"
 
 using namespace krq;
@@ -637,11 +638,19 @@ int balanced_grid(int64_t work, int64_t cap) {
 // =============================================================================================
 // C ABI
 // =============================================================================================
-// k_weight_lines' shapes: whole tiles, 16-byte aligned rows and copies, rows in registers.
-// Other shapes keep the one-row-per-workgroup kernels.
-static bool lines_ok(const void* w, int64_t N, int64_t K, int64_t ldw, const void* w8, const void* w8t) {
-  return N % 16 == 0 && K % 64 == 0 && K <= kLineMaxK && ldw % 8 == 0 && aligned16(w) && aligned16(w8) &&
-         aligned16(w8t);
+// k_weight_lines' shapes: whole tiles, 16-byte aligned rows and copies, rows in registers, and enough
+// rows (`least`): a workgroup of eight rows is a longer chain than one of a row, which pays once the
+// N / 8 workgroups cover the chip or the rows are short. One row per workgroup / lines, us, per channel
+// (one launch either way): K = 2,560 N = 512 4.95 / 5.28, 768 6.33 / 5.28; K = 4,096 N = 512 6.00 /
+// 6.29, 768 7.33 / 6.52; K = 16,384 N = 128 8.0 / 15.8, 768 16.3 / 17.6, 1,024 22.9 / 18.6. Per tensor
+// the lines are two launches for three, and a call outside a graph is as long as its launches up to
+// K = 10,240 (four weights of 16 rows, K = 2,560 to 9,728: 86 / 71); past that their longest variant is
+// longer than these (K = 16,384 N = 128 in a graph 14.3 / 23.1). Other shapes keep the
+// one-row-per-workgroup kernels.
+static bool lines_ok(const void* w, int64_t N, int64_t K, int64_t ldw, const void* w8, const void* w8t,
+                     int64_t least) {
+  return N >= std::min<int64_t>(1024, least) && N % 16 == 0 && K % 64 == 0 && K <= kLineMaxK && ldw % 8 == 0 &&
+         aligned16(w) && aligned16(w8) && aligned16(w8t);
 }
 
 template <int MODE>
@@ -668,7 +677,7 @@ extern "C" int krq_quant_fp8_rows(const void* w_bf16, int64_t N, int64_t K, int6
   KRQ_REQUIRE(!w8_tiled || (N % 16 == 0 && K % 64 == 0),
               "quant_fp8_rows: tiled layout needs N %% 16 == 0 and K %% 64 == 0 (N=%lld K=%lld)",
               (long long)N, (long long)K);
-  if (lines_ok(w_bf16, N, K, ldw, w8, w8_tiled)) {
+  if (lines_ok(w_bf16, N, K, ldw, w8, w8_tiled, 256 + K / 8)) {
     launch_weight_lines<0>(w_bf16, N, K, ldw, w8, w8_tiled, scale, nullptr, 0, static_cast<int>(N / 8),
                            (hipStream_t)stream);
     return krq_check_launch("quant_fp8_rows");
@@ -691,7 +700,7 @@ extern "C" int krq_quant_fp8_tensor(const void* w_bf16, int64_t N, int64_t K, in
               "quant_fp8_tensor: tiled layout needs N %% 16 == 0 and K %% 64 == 0 (N=%lld K=%lld)",
               (long long)N, (long long)K);
   hipStream_t s = (hipStream_t)stream;
-  if (lines_ok(w_bf16, N, K, ldw, w8, w8_tiled)) {
+  if (lines_ok(w_bf16, N, K, ldw, w8, w8_tiled, K > 10240 ? 1024 : 0)) {
     const int np = balanced_grid(N / 8, kLinePartials);  // (at most N / 8 partials, within row_amax_ws)
     launch_weight_lines<1>(w_bf16, N, K, ldw, nullptr, nullptr, nullptr, row_amax_ws, 0, np, s);
     launch_weight_lines<2>(w_bf16, N, K, ldw, w8, w8_tiled, scale0, row_amax_ws, np, static_cast<int>(N / 8), s);

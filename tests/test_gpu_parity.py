@@ -186,11 +186,14 @@ def test_quantize_per_channel(dev, N, K):
 
 
 # k_weight_lines: eight-row groups, 128-element pieces. K below one piece, a half last piece, the last
-# K of each register variant and the first of the next, a strided matrix, and (N or K not in whole tiles,
-# rows past its longest) the one-row kernels. Every row holds bf16 bit patterns of all magnitudes up to
-# its maximum, which runs over the binades, so quotients fall on both sides of the e4m3 midpoints.
-@pytest.mark.parametrize("N,K,pad", [(16, 64, 0), (48, 192, 8), (16, 1024, 0), (32, 1088, 0), (16, 2560, 64),
-                                     (16, 2624, 0), (16, 4096, 0), (16, 4160, 0), (16, 10240, 0), (16, 10304, 0),
+# K of each register variant and the first of the next, a strided matrix, at the fewest rows it takes per
+# channel; and (fewer rows, N or K not in whole tiles, rows past its longest) the one-row kernels. Every
+# row holds bf16 bit patterns of all magnitudes up to its maximum, which runs over the binades, so
+# quotients fall on both sides of the e4m3 midpoints.
+@pytest.mark.parametrize("N,K,pad", [(272, 64, 0), (288, 192, 8), (384, 1024, 0), (416, 1088, 0), (576, 2560, 64),
+                                     (592, 2624, 0), (768, 4096, 0), (784, 4160, 0), (1024, 10304, 0),
+                                     (1040, 16384, 0), (16, 64, 0), (48, 192, 8), (16, 1024, 0), (32, 1088, 0),
+                                     (16, 2560, 64), (16, 2624, 0), (16, 4096, 0), (16, 4160, 0), (16, 10240, 0), (16, 10304, 0),
                                      (16, 16384, 0), (16, 16448, 0), (24, 128, 0), (16, 72, 0), (16, 128, 4)])
 @pytest.mark.parametrize("per_tensor", [False, True])
 def test_quantize_lines(dev, N, K, pad, per_tensor):
