@@ -592,10 +592,11 @@ __global__ __launch_bounds__(kQT) void k_cast_pieces(const uint16_t* __restrict_
 
 // pass 2 folded into the cast (linear_fp8 without a given scale): every block reduces the g
 // partials itself (g <= kActPartials, 4 KB from L2), finishes the scale as k_act_fold does (block 0
-// stores amax, inv, scale) and casts its pieces with that inverse - the bytes of pass 2 then the
-// cast, one launch fewer. With a finite maximum and a headroom of at least one no product exceeds
-// 448.0001, which the convert takes to 448 as the clamp would.
-__global__ __launch_bounds__(kQT) void k_cast_fold_vec(const uint16_t* __restrict__ x, int64_t np,
+// stores amax, inv, scale) and casts its pieces with that inverse (and, with tail, the eight values
+// after them) - the bytes of pass 2 then the cast, one launch fewer. With a finite maximum and a
+// headroom of at least one no product exceeds 448.0001, which the convert takes to 448 as the clamp
+// would.
+__global__ __launch_bounds__(kQT) void k_cast_fold_vec(const uint16_t* __restrict__ x, int64_t np, int tail,
                                                        const float* __restrict__ ws, int g, float headroom,
                                                        float* amax, float* inv, float* scale,
                                                        uint8_t* __restrict__ x8) {
@@ -607,6 +608,7 @@ __global__ __launch_bounds__(kQT) void k_cast_fold_vec(const uint16_t* __restric
     amax[0] = a;
     inv[0] = iv;
     scale[0] = scale_from_amax(a);
+    if (tail) *reinterpret_cast<uint2*>(x8 + 16 * np) = quant8(ld16(reinterpret_cast<const uint8_t*>(x) + 32 * np), iv);
   }
   const bool own = finite_f32(a) && headroom >= 1.0f;
   cast_pieces(reinterpret_cast<const uint8_t*>(x), np, own, [&](int64_t) { return iv; }, x8);
@@ -771,10 +773,10 @@ extern "C" int krq_act_scale_cast_fp8(const void* x_bf16, int64_t M, int64_t K, 
   KRQ_REQUIRE(M > 0 && K > 0, "act_scale_cast: bad shape M=%lld K=%lld", (long long)M, (long long)K);
   hipStream_t s = (hipStream_t)stream;
   const int g = absmax_partials(x_bf16, M, K, ws, s);
-  if (vec_ok(x_bf16, K, K) && M * K % 16 == 0 && aligned16(x8)) {
+  if (vec_ok(x_bf16, K, K) && aligned16(x8)) {  // (M K a multiple of eight: whole pieces, or half of one more)
     const int gc = cast_grid(M * K / 16);
-    hipLaunchKernelGGL(k_cast_fold_vec, dim3(gc), dim3(kQT), 0, s, (const uint16_t*)x_bf16, M * K / 16, ws, g,
-                       headroom, amax, inv, scale, (uint8_t*)x8);
+    hipLaunchKernelGGL(k_cast_fold_vec, dim3(gc), dim3(kQT), 0, s, (const uint16_t*)x_bf16, M * K / 16,
+                       static_cast<int>(M * K % 16 != 0), ws, g, headroom, amax, inv, scale, (uint8_t*)x8);
   } else {  // the two passes and the cast
     hipLaunchKernelGGL(k_act_fold, dim3(1), dim3(1024), 0, s, ws, g, headroom, amax, inv, scale);
     return krq_cast_fp8(x_bf16, M, K, inv, 0, x8, stream);

@@ -105,7 +105,8 @@ def test_act_scale_and_cast(dev):
 # with a NaN or an infinity beside finite ones, products past 448 (headroom and inverses below the
 # maximum's), zero, negative, infinite and NaN inverses, per-row inverses, one piece, a partial last
 # round of pieces, and the eight-value (K % 16 == 8) and scalar kernels.
-@pytest.mark.parametrize("M,K", [(1, 16), (3, 2560), (17, 4112), (5, 200), (2, 100), (300, 9728)])
+@pytest.mark.parametrize("M,K", [(1, 8), (3, 8), (1, 16), (3, 2560), (17, 4112), (5, 200), (2, 100), (64, 16384),
+                                 (257, 4112), (300, 9728)])
 def test_cast_pieces(dev, M, K):
     x = act(M, K, 70 + M, 3.0)
     clean = x.to(dev)
