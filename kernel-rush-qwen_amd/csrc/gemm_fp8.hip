@@ -617,7 +617,12 @@ int gemm_run(const void* x, int x_kind, const float* x_scale, const float* x_inv
         // pair's latency per pair with two. Weights cold in the caches, two -> four buffers, us: M =
         // 64 QKV 11.1 -> 7.2, O 15.8 -> 9.4, down 14.2 -> 10.7; M = 256 O 15.8 -> 9.6, down 20.0 ->
         // 17.0; eight buffers (one workgroup per unit) measured 7.9, 9.3 and 11.1 at M = 64.
-        const bool deep = units <= (rp.bm == 64 ? 2 : 1) * (int64_t)cus;
+        // Not on a short K or a weight of under 2 MiB, whose bytes the caches hold and whose pairs are
+        // fewer than pay the longer start (128 x 256 2.96 / 3.21, 1,024 x 1,024 4.20 / 4.38, 12,288 x 512
+        // at M = 128 5.16 / 5.40; 8,192 x 1,024 at M = 64 6.11 / 4.66), nor with two tiles per unit of
+        // more than 1,024 rows (1,024 x 4,096 at M = 2,048 18.4 / 20.2).
+        const bool deep = units <= (rp.bm == 64 ? 2 : 1) * (int64_t)cus &&
+                          (K >= 2048 || (K >= 1024 && N * K >= (1 << 21))) && (units <= cus || M <= 1024);
 #define KRQ_RING_DEEP(BM_, OCC_, PART_)                            \
   if (deep) KRQ_RING(BM_, BM_, OCC_ / 2, PART_, 4, 0, N);          \
   else KRQ_RING(BM_, BM_, OCC_, PART_, 2, 0, N)

@@ -156,10 +156,13 @@ def test_linear_fp8_prefill_route(dev, M, N, K):
     assert rel_err(y.float().cpu().numpy(), ref) <= TOL
 
 
-# Four pair buffers: fewer pairs of stages than buffers (K = 256, 384), as many, one more; rows from
-# the first the GEMM takes, ragged and whole tiles; two 64 x 64 units per compute unit and one tile
-# more (N = 16,512: two buffers); 128 x 128 tiles, split K on either kind, one part per unit or past it.
-@pytest.mark.parametrize("M,N,K", [(33, 128, 256), (64, 128, 384), (77, 256, 512), (65, 384, 640), (127, 128, 1152),
+# Short K (two pair buffers: fewer pairs of stages than four, as many, one more) and four pair buffers from
+# K = 1,024 with 2 MiB of weights (one part on each side) or K = 2,048; rows from the first the GEMM
+# takes, ragged and whole tiles; two 64 x 64 units per compute unit up to 1,024 rows and past them, one
+# tile more (two buffers); 128 x 128 tiles, split K on either kind, one part per unit or past it.
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 1024), (100, 1920, 1024), (65, 128, 2048), (77, 1408, 1536),
+                                   (100, 16384, 2048), (100, 16512, 2048), (1000, 2048, 2048), (2048, 1024, 4096),
+                                   (33, 128, 256), (64, 128, 384), (77, 256, 512), (65, 384, 640), (127, 128, 1152),
                                    (100, 16384, 256), (100, 16512, 256), (33, 2560, 9728), (127, 2560, 9728),
                                    (129, 2560, 9728), (300, 2560, 8192), (200, 2560, 4096)])
 def test_gemm_deep_ring(dev, M, N, K):
