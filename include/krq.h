@@ -148,8 +148,9 @@ int krq_gemv_fp8(const void* x, int x_kind, const float* x_scale, const float* x
                  const void* w8, int w_layout, const float* w_scale, int w_per_row,
                  int64_t M, int64_t N, int64_t K, int split, int mode, int algo,
                  void* out, void* stream);
-/* 1 where krq_gemv_fp8 on KRQ_X_FP8_TILED rows (KRQ_OUT_BF16 or KRQ_OUT_PARTIAL, 2 <= M <= 16) runs
- * the launch whose workgroups share the rows in LDS, else 0: with it the tiled rows pay from fewer rows. */
+/* The workgroups of the launch that shares the rows in LDS where krq_gemv_fp8 on KRQ_X_FP8_TILED rows
+ * (KRQ_OUT_BF16 or KRQ_OUT_PARTIAL, 2 <= M <= 16) runs it, else 0: with it the tiled rows pay from
+ * fewer rows. */
 int64_t krq_gemv_fp8_shares_rows(int64_t M, int64_t N, int64_t K, int split, int w_layout);
 
 /*

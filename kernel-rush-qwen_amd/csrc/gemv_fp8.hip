@@ -745,7 +745,7 @@ extern "C" int64_t krq_gemv_fp8_shares_rows(int64_t M, int64_t N, int64_t K, int
   const int kts = static_cast<int>(K / split / 64);
   int u = 0, nw = 0;
   rows_ring((kts + 1) / 2, 1, &u, &nw);  // (krq_gemv_fp8's plan at M <= 16)
-  return wide32_shape(M, row_blocks(M, KRQ_OUT_BF16, 1, N, split), nw, N, kts);
+  return wide32_shape(M, row_blocks(M, KRQ_OUT_BF16, 1, N, split), nw, N, kts) ? N / 16 / kWideRb * split : 0;
 }
 
 extern "C" int krq_gemv_swiglu_fp8_cast(const void* x, int x_kind, const float* x_scale, const float* x_inv,

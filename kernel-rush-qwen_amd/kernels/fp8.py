@@ -351,19 +351,25 @@ def _activation_fp8(x, a, xs):
 # 7.52 / 7.40; gate_up M = 4 12.64 / 13.47, M = 16 14.19 / 13.70; down M = 4 9.70 / 10.35, M = 16
 # 11.24 / 10.83; given scale M = 8 QKV 7.19 / 7.60, M = 16 8.25 / 7.68, M = 32 10.47 / 9.29.
 TILED_MIN_ROWS = 13
-# Split-K GEMVs take the tiled rows earlier where their workgroups share them in LDS (k_gemv_wide32, as
-# krq_gemv_fp8_shares_rows tells): with a given scale from three rows, scaled per token from eleven
-# (QKV, O, gate_up and down of eight layers in one graph, row-major / tiled, us: given M = 2 273.8 /
-# 279.7, M = 3 291.5 / 282.4, M = 7 303.7 / 288.2; per token M = 9 284.8 / 287.1, M = 10 299.2 / 298.0,
-# M = 12 305.2 / 298.7). Launches that do not share them lose by the padding to sixteen rows: one K pass
-# over a whole row (linear_fp8 over a layer's four projections at M = 5 36.4 us row-major, 43.0 tiled),
-# weights without a tiled copy (down, given scale, M = 5 11.3 / 11.8, M = 8 11.7 / 12.0), N = 16 mod 64
-# (2,576 x 9,728, M = 5 8.9 / 9.5) and splits longer than LDS holds (2,560 x 16,384 in two, M = 5 14.2
-# / 16.1). Split-K launches of those kinds take the tiled rows from TILED_MIN_ROWS (M = 11 / 12 per token
-# 9.7 / 9.8 row-major, 10.0 / 10.0 tiled at 2,576 x 9,728), with a given scale from eleven (M = 11 without
-# a tiled copy: QKV 8.8 / 8.4, down 12.3 / 12.1).
+# Split-K GEMVs take the tiled rows earlier where the launch whose workgroups share them in LDS
+# (k_gemv_wide32; krq_gemv_fp8_shares_rows gives its workgroups) covers the chip. With a given scale,
+# row-major / tiled, us, from three rows while they are one round on 256 compute units: eight layers'
+# QKV (192 workgroups), O, down (160) and gate_up in one graph M = 2 273.8 / 279.7, M = 3 291.5 / 282.4,
+# M = 7 303.7 / 288.2; 5,120 x 5,120 in two (160) M = 3 8.44 / 8.49, M = 8 9.21 / 8.54. On fewer a unit
+# streams more (1,024 x 4,096 in four, 64, M = 5 5.02 / 5.64; 1,280 x 8,192 in two, 40, 7.23 / 9.58), on
+# more the padding to sixteen rows costs (8,192 x 8,192 in four, 512, M = 5 15.4 / 17.7): there from
+# eleven rows (11,008 x 4,096 in two, 344, M = 11 13.5 / 12.7, M = 5 12.2 / 12.6) and below 80
+# workgroups not at all (1,280 x 8,192 in two M = 11 7.65 / 9.65). Scaled per token from eleven
+# (the layers M = 9 284.8 / 287.1, M = 10 299.2 / 298.0, M = 12 305.2 / 298.7), by the same 80.
+# Launches that do not share the rows lose by the padding: one K pass over a whole row (linear_fp8 over
+# a layer's four projections at M = 5 36.4 us row-major, 43.0 tiled), weights without a tiled copy
+# (down, given scale, M = 5 11.3 / 11.8), N = 16 mod 64 (2,576 x 9,728, M = 5 8.9 / 9.5), long splits
+# (2,560 x 16,384 in two, M = 5 14.2 / 16.1). Split-K launches of those kinds take the tiled rows from
+# TILED_MIN_ROWS (M = 12 per token 9.8 / 10.0 at 2,576 x 9,728), with a given scale from eleven (M = 11
+# without a tiled copy: QKV 8.8 / 8.4, down 12.3 / 12.1).
 TILED_MIN_ROWS_SPLIT = {"given": 3, "token": 11}
 TILED_MIN_ROWS_SPLIT_APART = {"given": 11, "token": TILED_MIN_ROWS}
+TILED_SPLIT_MANY_ROWS, TILED_SPLIT_LEAST_GROUPS, TILED_SPLIT_ONE_ROUND = 11, 80, (144, 240)
 
 
 def _tiled_least(q, M, split, a):
@@ -372,8 +378,14 @@ def _tiled_least(q, M, split, a):
     if M < TILED_MIN_ROWS_SPLIT[kind]:
         return TILED_MIN_ROWS
     N, K = q[0].shape
-    shared = getattr(q, "tiled", None) is not None and L.lib().krq_gemv_fp8_shares_rows(M, N, K, split, L.W_TILED)
-    return (TILED_MIN_ROWS_SPLIT if shared else TILED_MIN_ROWS_SPLIT_APART)[kind]
+    tiled = getattr(q, "tiled", None) is not None
+    groups = L.lib().krq_gemv_fp8_shares_rows(M, N, K, split, L.W_TILED) if tiled else 0
+    if groups == 0:
+        return TILED_MIN_ROWS_SPLIT_APART[kind]
+    least, most = TILED_SPLIT_ONE_ROUND
+    if least <= groups <= most:
+        return TILED_MIN_ROWS_SPLIT[kind]
+    return TILED_SPLIT_MANY_ROWS if groups >= TILED_SPLIT_LEAST_GROUPS else TILED_MIN_ROWS
 
 
 def _tiled_rows(x, M, K, a, xs, algo, least=TILED_MIN_ROWS):

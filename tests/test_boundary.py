@@ -268,8 +268,8 @@ def test_tiled_rows_only_where_shared():
     head's persistent launch on a grid that fills the chip."""
     lib = L.lib()
     shares = lib.krq_gemv_fp8_shares_rows
-    assert shares(5, 6144, 2560, 2, L.W_TILED) == shares(16, 2560, 9728, 4, L.W_TILED) == 1
-    assert shares(3, 65536, 1024, 2, L.W_TILED) == 1 and shares(5, 65536, 1024, 2, L.W_TILED) == 0  # (paired above 4 rows)
+    assert shares(5, 6144, 2560, 2, L.W_TILED) == 192 and shares(16, 2560, 9728, 4, L.W_TILED) == 160
+    assert shares(3, 65536, 1024, 2, L.W_TILED) == 2048 and shares(5, 65536, 1024, 2, L.W_TILED) == 0  # (paired above 4)
     for bad in ((5, 6144, 2560, 2, L.W_ROWMAJOR), (5, 6160, 2560, 2, L.W_TILED), (5, 2560, 16384, 2, L.W_TILED),
                 (5, 6144, 2560, 3, L.W_TILED), (5, 6144, 2592, 2, L.W_TILED), (1, 6144, 2560, 2, L.W_TILED),
                 (17, 6144, 2560, 2, L.W_TILED), (5, 0, 2560, 2, L.W_TILED), (5, 6144, 2560, 0, L.W_TILED)):
@@ -287,7 +287,8 @@ def test_tiled_rows_only_where_shared():
     for scale, least, apart in ((a, 3, 11), (None, 11, 13)):
         for M in range(1, 13):
             for q, want in ((fp8.FP8Weight(w8, t, t), least), (fp8.FP8Weight(w8, t, None), apart), ((w8, t), apart),
-                            (fp8.FP8Weight(w8[:2544], t, t), apart)):
+                            (fp8.FP8Weight(w8[:2544], t, t), apart), (fp8.FP8Weight(w8[:1280], t, t), 11),
+                            (fp8.FP8Weight(w8[:1216], t, t), 13), (fp8.FP8Weight(w8.expand(2, -1, -1).reshape(-1, 9728), t, t), 11)):
                 assert (M >= fp8._tiled_least(q, M, 4, scale)) == (M >= want)
 
 

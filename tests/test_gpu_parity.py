@@ -987,7 +987,8 @@ def test_picked_cast_is_used(dev, M, monkeypatch):
 # Split-K rows below TILED_MIN_ROWS on weights whose launch does not share them (no tiled copy, N = 16 mod
 # 64) and on those whose launch does: one product, whatever the route.
 @pytest.mark.parametrize("M", [3, 5, 10, 11, 12, 13])
-@pytest.mark.parametrize("N,K,split,tiled", [(256, 1024, 2, False), (272, 1024, 2, True), (256, 1024, 2, True)])
+@pytest.mark.parametrize("N,K,split,tiled", [(256, 1024, 2, False), (272, 1024, 2, True), (256, 1024, 2, True),
+                                             (6144, 256, 2, True), (16384, 128, 2, True)])
 def test_split_rows_routes(dev, M, N, K, split, tiled):
     x, w = act(M, K, 100 + M).to(dev), weight(N, K, 101).to(dev)
     q, ref = fp8.quantize(w, tiled=tiled), fp8.quantize(w, tiled=False)
@@ -996,5 +997,9 @@ def test_split_rows_routes(dev, M, N, K, split, tiled):
         x8, xs = (fp8.quant_rows(x) if s is None else (fp8._cast_hip(x, s), s.scale))
         want = fp8.gemv_fp8_launch(x8, xs, ref, split, L.OUT_PARTIAL)
         assert torch.equal(fp8.gemv_fp8(x, q, split, s), want)
+        if M < fp8.TILED_MIN_ROWS:  # (rows off 16 bytes keep the row-major quantizers)
+            off = torch.empty(M * K + 1, dtype=torch.bfloat16, device=dev)[1:].view(M, K)
+            off.copy_(x)
+            assert torch.equal(fp8.gemv_fp8(off, q, split, s), want)
         _, yref = O.fp8_matmul(u8(x8), xs.cpu().numpy().reshape(-1), u8(ref[0]), ref[1].cpu().numpy())
         assert rel_err(want.sum(0).cpu().numpy(), yref) <= TOL
