@@ -13,6 +13,11 @@ using namespace krq;
 
 namespace {
 
+// How a block's operands are loaded: in the tiles' lane order (64 bytes of sixteen rows per load), in
+// whole lines of eight rows that lanes exchange into the tiles' operands (row-major weights too), or so
+// with one activation load per step (at most eight rows).
+constexpr int kTileLoads = 0, kLineLoads = 1, kOneLine = 2;
+
 // PB = 2 or 4: adjacent row blocks per block sharing the activation loads (as in gemv_fp8.hip;
 // 4 for the multi-row lm_head, where every 16-column block re-reads the bf16 rows from L2).
 // bx: the column block this workgroup owns (its two-matrix, paired or single row block, or with
@@ -23,7 +28,7 @@ namespace {
 // that gives up makes the block's partials NaN) and then reads act with agent-scope (sc1) loads,
 // and counts its exit. sy >= 0 / nwo > 0: the block's K split and its wave count, given (the
 // chained kernel's one-dimensional grid and common block size); waves past nwo end at once.
-template <int MT, int MODE, int LAYOUT, int ALGO, int U, int PB, bool XO, bool CHAIN = false>
+template <int MT, int MODE, int LAYOUT, int ALGO, int U, int PB, int XM, bool CHAIN = false>
 KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __restrict__ w, int M, int64_t NO,
                             int64_t K, int kts, void* __restrict__ out, void* __restrict__ aux, int64_t bx,
                             int sy = -1, int nwo = 0, const FusedArgs* fa = nullptr) {
@@ -31,7 +36,9 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
   __shared__ float ones[32];
   static_assert(PB == 1 || (MODE != KRQ_OUT_SWIGLU && ALGO != 2), "paired row blocks: MFMA, no SwiGLU");
   static_assert(PB == 1 || PB == 2 || PB == 4, "one, two or four row blocks per block");
-  static_assert(XO ? MT == 1 : ALGO != 2 || LAYOUT == KRQ_W_TILED, "one activation load per step: at most eight rows");
+  constexpr bool XO = XM == kOneLine;
+  static_assert(!XO || MT == 1, "one activation load per step: at most eight rows");
+  static_assert(ALGO != 2 || XM == kTileLoads || (XO && LAYOUT == KRQ_W_ROWMAJOR), "one row: no lines on packed weights");
   static_assert(!CHAIN || (PB == 1 && (MODE == KRQ_OUT_SWIGLU || MODE == kOutSwiGluHalf || MODE == KRQ_OUT_PARTIAL)),
                 "chained MLP: SwiGLU first stage, partials second stage");
   constexpr bool WAITS = CHAIN && MODE == KRQ_OUT_PARTIAL;  // (second stage)
@@ -46,7 +53,7 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
   const int64_t tbase = (int64_t)sidx * kts;
   const int64_t rowb = 2 * K;
   const int jcount = wave < nsteps ? (nsteps - wave + nw - 1) / nw : 0;
-  constexpr bool RM = LAYOUT == KRQ_W_ROWMAJOR;  // loads of whole lines (w_line_chunk)
+  constexpr bool RM = LAYOUT == KRQ_W_ROWMAJOR && XM != kTileLoads;  // weights in whole lines (w_line_chunk)
   if (threadIdx.x < 32) ones[threadIdx.x] = 1.0f;
   // weight set p: the up half of the SwiGLU, else the p-th row block of this block
   auto rbp = [&](int p) -> int64_t { return MODE == KRQ_OUT_SWIGLU && p == 1 ? rb + (NO >> 4) : rb + p; };
@@ -91,11 +98,9 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
       }
     }
   };
-  // The activations in whole lines too (XL), row by row as row-major weights; XO: one load per step, the
-  // lane columns c and c + 8 taking the two halves of row c's line.
-  // (Not for four row blocks of tiled weights, the head's launch at 5-16 rows, where the exchange costs
-  // more than the half lines: V = 151,936, M = 8 142.3 -> 135.2 us, M = 16 148.8 -> 144.3.)
-  constexpr bool XL = RM || (ALGO != 2 && PB != 4);
+  // The activations in whole lines too, row by row as row-major weights; XO: one load per step, the lane
+  // columns c and c + 8 taking the two halves of row c's line.
+  constexpr bool XL = XM != kTileLoads;
   auto load_x = [&](int u, int cc) {
     const int j = jcount > 0 ? wave + min(cc, jcount - 1) * nw : 0;
     const int64_t t0 = tbase + 2 * j;
@@ -151,7 +156,7 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
     for (int p = 0; p < P; ++p) {
       uint4 bl = wl[p][u], bh = wh[p][u];
       if constexpr (RM) lines_to_tiles(wl[p][u], wh[p][u], &bl, &bh);
-      if constexpr (!SKIP) {
+      if constexpr (LAST && !SKIP) {
         bl = sel4(ok, bl);
         bh = sel4(hi, bh);
       }
@@ -255,12 +260,12 @@ KRQ_DEV void gemv_bf16_body(const uint8_t* __restrict__ x, const uint8_t* __rest
   if constexpr (CHAIN) chain_tail<!WAITS>(*fa);
 }
 
-template <int MT, int MODE, int LAYOUT, int ALGO, int U, int PB, bool XO = false>
+template <int MT, int MODE, int LAYOUT, int ALGO, int U, int PB, int XM>
 __global__ __launch_bounds__(512) void k_gemv_bf16(const uint8_t* __restrict__ x,
                                                   const uint8_t* __restrict__ w, int M, int64_t NO,
                                                   int64_t K, int kts, void* __restrict__ out,
                                                   void* __restrict__ aux) {
-  gemv_bf16_body<MT, MODE, LAYOUT, ALGO, U, PB, XO>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
+  gemv_bf16_body<MT, MODE, LAYOUT, ALGO, U, PB, XM>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
 }
 
 // Wide blocks at 4 < M <= 32: a workgroup of four waves owns four adjacent row blocks (one per wave, 64
@@ -413,15 +418,15 @@ __global__ __launch_bounds__(kWideRb * 64) void k_gemv_bf16_wide(const uint8_t* 
 // The SwiGLU with its last column blocks split in half, as k_gemv_fp8_swiglu_mixed: workgroups
 // below nfull are two-matrix blocks, workgroup nfull + j is half-pair block 2 nfull + j (the same
 // steps per wave, so the same output bits).
-template <int LAYOUT, int ALGO, int U, bool XO = false>
+template <int LAYOUT, int ALGO, int U, int XM>
 __global__ __launch_bounds__(512) void k_gemv_bf16_swiglu_mixed(const uint8_t* __restrict__ x,
                                                                const uint8_t* __restrict__ w, int M, int64_t NO,
                                                                int64_t K, int kts, void* __restrict__ out,
                                                                void* __restrict__ aux, int nfull) {
   if (static_cast<int>(blockIdx.x) < nfull)
-    gemv_bf16_body<1, KRQ_OUT_SWIGLU, LAYOUT, ALGO, U, 1, XO>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
+    gemv_bf16_body<1, KRQ_OUT_SWIGLU, LAYOUT, ALGO, U, 1, XM>(x, w, M, NO, K, kts, out, aux, blockIdx.x);
   else
-    gemv_bf16_body<1, kOutSwiGluHalf, LAYOUT, ALGO, U, 1, XO>(x, w, M, NO, K, kts, out, aux,
+    gemv_bf16_body<1, kOutSwiGluHalf, LAYOUT, ALGO, U, 1, XM>(x, w, M, NO, K, kts, out, aux,
                                                           (int64_t)blockIdx.x + nfull);
 }
 
@@ -432,7 +437,7 @@ __global__ __launch_bounds__(512) void k_gemv_bf16_swiglu_mixed(const uint8_t* _
 // of K split p / nrb2. Each stage keeps the standalone launch's plan, so act and the partials are
 // those of the two launches, bit for bit. The block holds max(NWG, NWD) waves; the waves a stage
 // does not use end at once (a barrier waits only for the waves that have not ended).
-template <int MT, int LAYOUT, int ALGO, int U, bool XO>
+template <int MT, int LAYOUT, int ALGO, int U, int XM>
 __global__ __launch_bounds__(512) void k_mlp_chain_bf16(const uint8_t* __restrict__ x, const uint8_t* __restrict__ wgu,
                                                        const uint8_t* __restrict__ wd, int M, int64_t I, int64_t H,
                                                        int kts_g, int kts_d, int nfull, int nrb2, int nwg, int nwd,
@@ -440,14 +445,14 @@ __global__ __launch_bounds__(512) void k_mlp_chain_bf16(const uint8_t* __restric
                                                        FusedArgs fa) {
   const int w = static_cast<int>(blockIdx.x);
   if (w < nfull) {
-    gemv_bf16_body<MT, KRQ_OUT_SWIGLU, LAYOUT, ALGO, U, 1, XO, true>(x, wgu, M, I, H, kts_g, act, nullptr, w, 0, nwg, &fa);
+    gemv_bf16_body<MT, KRQ_OUT_SWIGLU, LAYOUT, ALGO, U, 1, XM, true>(x, wgu, M, I, H, kts_g, act, nullptr, w, 0, nwg, &fa);
   } else if (w < fa.n_first) {
     if constexpr (MT == 1)
-      gemv_bf16_body<1, kOutSwiGluHalf, LAYOUT, ALGO, U, 1, XO, true>(x, wgu, M, I, H, kts_g, act, nullptr,
+      gemv_bf16_body<1, kOutSwiGluHalf, LAYOUT, ALGO, U, 1, XM, true>(x, wgu, M, I, H, kts_g, act, nullptr,
                                                                   (int64_t)w + nfull, 0, nwg, &fa);
   } else {
     const int p = w - fa.n_first;
-    gemv_bf16_body<MT, KRQ_OUT_PARTIAL, LAYOUT, ALGO, U, 1, XO, true>(reinterpret_cast<const uint8_t*>(act), wd, M, H, I,
+    gemv_bf16_body<MT, KRQ_OUT_PARTIAL, LAYOUT, ALGO, U, 1, XM, true>(reinterpret_cast<const uint8_t*>(act), wd, M, H, I,
                                                                   kts_d, part, nullptr, p % nrb2, p / nrb2, nwd, &fa);
   }
 }
@@ -563,36 +568,39 @@ __global__ __launch_bounds__(512) void k_gemv_bf16_rows(const uint8_t* __restric
   }
 }
 
-template <int MODE, int LAYOUT>
+template <int MODE, int LAYOUT, bool LINES>
 void launch(int M, int pb, dim3 grid, int nw, size_t smem, hipStream_t s, const uint8_t* x,
             const uint8_t* w, int m, int64_t NO, int64_t K, int kts, void* out, void* aux) {
   const dim3 block(nw * 64);
   constexpr int PB2 = MODE == KRQ_OUT_SWIGLU ? 1 : 2;
   constexpr int PB4 = MODE == kOutArgmax ? 4 : 1;  // (pb is 4 only for the argmax epilogue)
   constexpr bool RM = LAYOUT == KRQ_W_ROWMAJOR;
-  if (M == 1)
-    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 2, 4, 1, RM>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
-  else if (M <= 4)
-    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 1, 4, 1, true>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
-  else if (M <= 16 && pb == 4)
-    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 1, 2, PB4>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
-  else if (M <= 16 && pb == 2)
-    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 1, 2, PB2>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
-  else if (M <= 16)
-    hipLaunchKernelGGL((k_gemv_bf16<1, MODE, LAYOUT, 1, 2, 1>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
-  else if (pb == 2)
-    hipLaunchKernelGGL((k_gemv_bf16<2, MODE, LAYOUT, 1, 2, PB2>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
-  else
-    hipLaunchKernelGGL((k_gemv_bf16<2, MODE, LAYOUT, 1, 2, 1>), grid, block, smem, s, x, w, m, NO, K, kts, out, aux);
+  constexpr int ONE = LINES ? kOneLine : kTileLoads, X = LINES ? kLineLoads : kTileLoads;
+#define KRQ_BF16(MT_, ALGO_, U_, PB_, XM_)                                                                           \
+  hipLaunchKernelGGL((k_gemv_bf16<MT_, MODE, LAYOUT, ALGO_, U_, PB_, XM_>), grid, block, smem, s, x, w, m, NO, K, kts, \
+                     out, aux)
+  if (M == 1) KRQ_BF16(1, 2, 4, 1, (RM ? ONE : kTileLoads));
+  else if (M <= 4) KRQ_BF16(1, 1, 4, 1, ONE);
+  else if (M <= 16 && pb == 4) KRQ_BF16(1, 1, 2, PB4, (RM ? X : kTileLoads));
+  else if (M <= 16 && pb == 2) KRQ_BF16(1, 1, 2, PB2, X);
+  else if (M <= 16) KRQ_BF16(1, 1, 2, 1, X);
+  else if (pb == 2) KRQ_BF16(2, 1, 2, PB2, X);
+  else KRQ_BF16(2, 1, 2, 1, X);
+#undef KRQ_BF16
 }
 
 template <int MODE>
-void launch_layout(int layout, int M, int pb, dim3 grid, int nw, size_t smem, hipStream_t s, const uint8_t* x,
+void launch_layout(int layout, bool lines, int M, int pb, dim3 grid, int nw, size_t smem, hipStream_t s, const uint8_t* x,
                    const uint8_t* w, int m, int64_t NO, int64_t K, int kts, void* out, void* aux) {
-  if (layout == KRQ_W_TILED)
-    launch<MODE, KRQ_W_TILED>(M, pb, grid, nw, smem, s, x, w, m, NO, K, kts, out, aux);
-  else
-    launch<MODE, KRQ_W_ROWMAJOR>(M, pb, grid, nw, smem, s, x, w, m, NO, K, kts, out, aux);
+#define KRQ_BF16_LAYOUT(LAYOUT_)                                                                        \
+  if (lines) launch<MODE, LAYOUT_, true>(M, pb, grid, nw, smem, s, x, w, m, NO, K, kts, out, aux);       \
+  else launch<MODE, LAYOUT_, false>(M, pb, grid, nw, smem, s, x, w, m, NO, K, kts, out, aux)
+  if (layout == KRQ_W_TILED) {
+    KRQ_BF16_LAYOUT(KRQ_W_TILED);
+  } else {
+    KRQ_BF16_LAYOUT(KRQ_W_ROWMAJOR);
+  }
+#undef KRQ_BF16_LAYOUT
 }
 
 constexpr int64_t kCUs = 256;  // compute units of the MI355X (workgroup b runs on CU b mod 256)
@@ -600,44 +608,77 @@ constexpr int64_t kCUs = 256;  // compute units of the MI355X (workgroup b runs 
 // k_gemv_bf16_swiglu_mixed for M <= 16 when the SwiGLU's column blocks number a little over a
 // multiple of the CUs (gate_up: 608 = 2 x 256 + 96), with the variant launch() would pick; false
 // otherwise.
-bool launch_swiglu_mixed(int layout, int M, int64_t NO, int nw, size_t smem, hipStream_t s, const uint8_t* x,
+bool launch_swiglu_mixed(int layout, bool lines, int M, int64_t NO, int nw, size_t smem, hipStream_t s, const uint8_t* x,
                          const uint8_t* w, int64_t K, int kts, void* out) {
   const int64_t nrbs = NO / 16, rem = nrbs % kCUs;
   if (M > 16 || nrbs <= 2 * kCUs || rem == 0 || 2 * rem > kCUs) return false;
   const int nfull = static_cast<int>(nrbs - rem);
   const dim3 grid(static_cast<unsigned>(nfull + 2 * rem), 1), block(nw * 64);
-#define KRQ_BF16_MIXED(LAYOUT)                                                                                   \
-  if (M == 1)                                                                                                    \
-    hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT, 2, 4, LAYOUT == KRQ_W_ROWMAJOR>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
-                       nullptr, nfull);                                                                          \
-  else if (M <= 4)                                                                                               \
-    hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT, 1, 4, true>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
-                       nullptr, nfull);                                                                          \
-  else                                                                                                           \
-    hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT, 1, 2>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
-                       nullptr, nfull);
+#define KRQ_MIXED(LAYOUT_, ALGO_, U_, XM_)                                                                          \
+  hipLaunchKernelGGL((k_gemv_bf16_swiglu_mixed<LAYOUT_, ALGO_, U_, XM_>), grid, block, smem, s, x, w, M, NO, K, kts, out, \
+                     nullptr, nfull)
+#define KRQ_MIXED_M(LAYOUT_, ONE_, ONE1_, X_)      \
+  if (M == 1) KRQ_MIXED(LAYOUT_, 2, 4, ONE1_);     \
+  else if (M <= 4) KRQ_MIXED(LAYOUT_, 1, 4, ONE_); \
+  else KRQ_MIXED(LAYOUT_, 1, 2, X_)
   if (layout == KRQ_W_TILED) {
-    KRQ_BF16_MIXED(KRQ_W_TILED)
+    if (lines) { KRQ_MIXED_M(KRQ_W_TILED, kOneLine, kTileLoads, kLineLoads); }
+    else { KRQ_MIXED_M(KRQ_W_TILED, kTileLoads, kTileLoads, kTileLoads); }
   } else {
-    KRQ_BF16_MIXED(KRQ_W_ROWMAJOR)
+    if (lines) { KRQ_MIXED_M(KRQ_W_ROWMAJOR, kOneLine, kOneLine, kLineLoads); }
+    else { KRQ_MIXED_M(KRQ_W_ROWMAJOR, kTileLoads, kTileLoads, kTileLoads); }
   }
-#undef KRQ_BF16_MIXED
+#undef KRQ_MIXED_M
+#undef KRQ_MIXED
   return true;
 }
 
+// Whether 16-column blocks (`blocks` of them, ks elements of K each) load whole lines. On row-major weights
+// a line then goes through the caches once instead of twice, on packed ones the activations do, but
+// the lanes' exchange lengthens every step of a block: it pays where the caches bound a unit's blocks,
+// not where one or two blocks' own chain does. Measured, us, tile loads / lines:
+//   row-major  QKV in two M = 1 10.7 / 8.3; 1,024 x 1,024 in four M = 1 3.33 / 3.53 (short chains); 5,120 x
+//              5,120 M = 6 22.0 / 16.6, but 4,096 x 4,096, one block per unit, 9.84 / 11.0
+//   SwiGLU     (two matrices a block) 8,192 x 8,192, 256 blocks, M = 6 33.4 / 36.9; gate_up M = 1 26.6 / 19.1;
+//              5,120 x 5,120, 160 blocks, M = 1 23.3 / 22.6, M = 24 27.6 / 26.5, M = 32 30.6 / 26.9;
+//              4,096 x 11,008, 128 blocks, M = 24 49.4 / 50.8, M = 32 55.1 / 51.8
+//   packed     up to 9 rows no gain (4,096 x 4,096 M = 6 8.9 / 9.7); 5,120 x 5,120 M = 12 15.7 / 14.8, M = 16
+//              18.2 / 16.6; one block per unit 4,096 x 4,096 M = 16 9.1 / 9.9, 4,096 x 11,008 M = 32 31.1 / 28.4;
+//              SwiGLU 4,096 x 4,096 M = 16 15.1 / 16.7, gate_up M = 12 19.2 / 18.5, 28,672 x 4,096 M = 8 40.2 /
+//              39.4, 11,008 x 4,096 (344 blocks) M = 24 25.2 / 24.4
+bool line_loads(int layout, int M, int mode, int64_t blocks, int64_t ks) {
+  const bool even = blocks == kCUs || blocks == 2 * kCUs;
+  if (layout == KRQ_W_ROWMAJOR) {
+    if (mode == KRQ_OUT_SWIGLU) return blocks >= (M > 24 ? 128 : M > 16 || M == 1 ? 160 : kCUs + 1);
+    return (ks >= 1280 || blocks >= 2 * kCUs) && !(even && M > 4 && M <= 8);
+  }
+  if (mode == KRQ_OUT_SWIGLU) return M >= 8 && blocks > (M > 16 ? kCUs : 2 * kCUs);
+  return M >= 10 && (M > 16 || !even);
+}
+
 // k_gemv_bf16_wide where it applies (false otherwise): launches of more than four rows whose replaced
-// plan has two waves, whole groups of four row blocks on at least half the compute units, the split's
+// plan has two waves, whole groups of four row blocks on half the compute units or more, the split's
 // activation rows within LDS. Four Qwen3-4B layers in one graph, us, 16-column blocks / wide, row-major
 // weights: M = 3 194.1 / 195.5 and M = 4 199.1 / 197.6 (left narrow), M = 6 202 / 190, M = 16 246 / 221,
-// M = 32 336 / 256; packed: M = 16 205 / 189, M = 32 291 / 229. Four slots: two measured 254 at M = 16 row-major, six 228, eight 234. The two-matrix
-// SwiGLU block (152 workgroups for gate_up) is wide above 16 rows only: at M = 16 23.8 us against
-// 25.2 wide, at M = 32 34.0 against 21.
+// M = 32 336 / 256; packed: M = 16 205 / 189, M = 32 291 / 229. Four slots: two measured 254 at M = 16
+// row-major, six 228, eight 234. The two-matrix SwiGLU block (152 workgroups for gate_up) is wide above
+// 16 rows only: at M = 16 23.8 us against 25.2 wide, at M = 32 34.0 against 21.
+// Fewer rows bring fewer activation bytes to share, and a grid a little over the units leaves most of a
+// second round empty. Packed up to 16 rows: not on half the units (4,096 x 4,096 in two M = 16 9.0 / 9.8, but
+// 8,192 x 1,024 M = 24 8.02 / 6.86), splits of at most 48 steps (LDS for two workgroups a unit; 8,192 x
+// 8,192 in two M = 6 22.7 / 25.9), and up to 12 within one round or on short splits (4,096 x 4,096 in four
+// M = 6 7.8 / 9.0, QKV in four 8.55 / 7.72). Row-major up to eight rows: not on half the units (8,192 x 8,192 M = 6 31.0 / 35.8) nor a
+// little over them (19,456 x 2,560, 304 workgroups, M = 6 22.4 / 25.0).
 bool launch_wide(int layout, int M, int mode, int pb, int nw, int64_t NO, int split, hipStream_t s, const uint8_t* x,
                  const uint8_t* w, int64_t K, int kts, void* out) {
-  const int64_t groups = NO / 16 / kWideRb;
-  const int kib = (kts + 1) / 2 * ((M + 7) / 8);  // LDS for the split's activation rows
-  if (M <= 4 || pb != 1 || nw != 2 || (NO / 16) % kWideRb != 0 || 2 * groups * split < kCUs || kib > 160)
+  const int64_t groups = NO / 16 / kWideRb, wgs = groups * split;
+  const int steps = (kts + 1) / 2, kib = steps * ((M + 7) / 8);  // LDS for the split's activation rows
+  if (M <= 4 || pb != 1 || nw != 2 || (NO / 16) % kWideRb != 0 || 2 * wgs < kCUs || kib > 160) return false;
+  if (layout == KRQ_W_TILED) {
+    if (M <= 16 && (wgs < 144 || steps > 48 || (M <= 12 && wgs > 240 && steps > 10))) return false;
+  } else if (M <= 8 && (wgs < 144 || (wgs > kCUs && wgs < 344))) {
     return false;
+  }
   if (M * 2 * K > 0x7fffffff) return false;  // (32-bit activation offsets)
   const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(split)), block(kWideRb * 64);
 #define KRQ_WIDE(MODE_, LAYOUT_, MT_, TL_) \
@@ -702,13 +743,14 @@ int krq::gemv_bf16_run(const void* x, const void* w, int w_layout, int64_t M, in
   const uint8_t* wb = (const uint8_t*)w;
   const int m = static_cast<int>(M);
   hipStream_t s = (hipStream_t)stream;
+  const bool lines = line_loads(w_layout, m, mode, NO / 16 * split, K / split);
   if (launch_wide(w_layout, m, mode, pb, nw, NO, split, s, xb, wb, K, kts, out)) return krq_check_launch("gemv_bf16");
-  if (mode == KRQ_OUT_BF16) launch_layout<KRQ_OUT_BF16>(w_layout, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
-  else if (mode == KRQ_OUT_PARTIAL) launch_layout<KRQ_OUT_PARTIAL>(w_layout, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
-  else if (mode == KRQ_OUT_SWIGLU && launch_swiglu_mixed(w_layout, m, NO, nw, smem, s, xb, wb, K, kts, out))
+  if (mode == KRQ_OUT_BF16) launch_layout<KRQ_OUT_BF16>(w_layout, lines, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
+  else if (mode == KRQ_OUT_PARTIAL) launch_layout<KRQ_OUT_PARTIAL>(w_layout, lines, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
+  else if (mode == KRQ_OUT_SWIGLU && launch_swiglu_mixed(w_layout, lines, m, NO, nw, smem, s, xb, wb, K, kts, out))
     ;  // the mixed launch below 17 rows on grids a little over a multiple of the CUs
-  else if (mode == KRQ_OUT_SWIGLU) launch_layout<KRQ_OUT_SWIGLU>(w_layout, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
-  else launch_layout<kOutArgmax>(w_layout, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
+  else if (mode == KRQ_OUT_SWIGLU) launch_layout<KRQ_OUT_SWIGLU>(w_layout, lines, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
+  else launch_layout<kOutArgmax>(w_layout, lines, m, pb, grid, nw, smem, s, xb, wb, m, NO, K, kts, out, aux);
   return krq_check_launch("gemv_bf16");
 }
 
@@ -794,14 +836,14 @@ extern "C" int krq_mlp_chain_bf16(const void* x, const void* w_gu, const void* w
   const uint8_t* gb = (const uint8_t*)w_gu;
   const uint8_t* db = (const uint8_t*)w_down;
   const int m = static_cast<int>(M);
-#define KRQ_CHAIN(MT_, LAYOUT, ALGO, U_, XO_)                                                                        \
-  hipLaunchKernelGGL((k_mlp_chain_bf16<MT_, LAYOUT, ALGO, U_, XO_>), grid, block, smem, s, xb, gb, db, m, I, H, kts_g, \
+#define KRQ_CHAIN(MT_, LAYOUT, ALGO, U_, XM_)                                                                        \
+  hipLaunchKernelGGL((k_mlp_chain_bf16<MT_, LAYOUT, ALGO, U_, XM_>), grid, block, smem, s, xb, gb, db, m, I, H, kts_g, \
                      kts_d, static_cast<int>(nfull), static_cast<int>(nrb2), nwg, nwd, (uint16_t*)act, (float*)out, fa)
-#define KRQ_CHAIN_M(LAYOUT)                          \
-  if (M == 1) KRQ_CHAIN(1, LAYOUT, 2, 4, LAYOUT == KRQ_W_ROWMAJOR);            \
-  else if (M <= 4) KRQ_CHAIN(1, LAYOUT, 1, 4, true);       \
-  else if (M <= 16) KRQ_CHAIN(1, LAYOUT, 1, 2, false);      \
-  else KRQ_CHAIN(2, LAYOUT, 1, 2, false);
+#define KRQ_CHAIN_M(LAYOUT)                                                                     \
+  if (M == 1) KRQ_CHAIN(1, LAYOUT, 2, 4, (LAYOUT == KRQ_W_ROWMAJOR ? kOneLine : kTileLoads));   \
+  else if (M <= 4) KRQ_CHAIN(1, LAYOUT, 1, 4, kOneLine);                                        \
+  else if (M <= 16) KRQ_CHAIN(1, LAYOUT, 1, 2, kLineLoads);                                     \
+  else KRQ_CHAIN(2, LAYOUT, 1, 2, kLineLoads);
   if (w_layout == KRQ_W_TILED) {
     KRQ_CHAIN_M(KRQ_W_TILED)
   } else {

@@ -1003,3 +1003,30 @@ def test_split_rows_routes(dev, M, N, K, split, tiled):
             assert torch.equal(fp8.gemv_fp8(off, q, split, s), want)
         _, yref = O.fp8_matmul(u8(x8), xs.cpu().numpy().reshape(-1), u8(ref[0]), ref[1].cpu().numpy())
         assert rel_err(want.sum(0).cpu().numpy(), yref) <= TOL
+
+
+# Every load variant of the BF16 blocks (tile loads, whole lines, one line) on either side of its lines: short
+# and long K per block, one and two blocks per compute unit, a little over, the SwiGLU's 128, 160, 256 and
+# 512 blocks, wide workgroups on half the units, one round, a little over and past it. Row-major weights and
+# their packed copy give one result.
+@pytest.mark.parametrize("M", [1, 3, 6, 7, 8, 9, 10, 12, 13, 16, 17, 24, 25, 32])
+@pytest.mark.parametrize("N,K,split,swiglu", [(256, 1248, 1, False), (256, 1280, 1, False), (4096, 1280, 1, False),
+                                              (4096, 1344, 2, False), (8192, 96, 1, False), (8208, 96, 1, False),
+                                              (4096, 768, 4, False), (4864, 2176, 4, False), (5632, 768, 4, False),
+                                              (2304, 3200, 4, False), (2304, 12416, 4, False),
+                                              (4064, 160, 1, True), (4096, 160, 1, True), (5088, 160, 1, True), (5120, 160, 1, True),
+                                              (8192, 160, 1, True), (8224, 160, 1, True), (16384, 96, 1, True),
+                                              (16416, 96, 1, True)])
+def test_bf16_load_variants(dev, M, N, K, split, swiglu):
+    from kernels import gemv as G
+    x, w = act(M, K, 110 + M).to(dev), weight(N, K, 111).to(dev)
+    run = (lambda: G.gemv_swiglu(x, w)) if swiglu else (lambda: G.gemv(x, w, split))
+    y = run()
+    G.pack(w)
+    assert torch.equal(run(), y)
+    ref = x.double() @ w.double().t()
+    if swiglu:
+        g, u = ref[:, :N // 2].to(torch.bfloat16).double(), ref[:, N // 2:].to(torch.bfloat16).double()
+        ref = torch.nn.functional.silu(g).to(torch.bfloat16).double() * u
+    got = y.double().sum(0) if split > 1 else y.double()
+    assert rel_err(got.cpu(), ref.cpu()) <= TOL
